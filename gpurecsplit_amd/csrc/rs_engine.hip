@@ -498,27 +498,23 @@ static void launch_kind(hipStream_t s, const uint64_t *keys, const SearchArgs &a
                         size_t lds) {
     if constexpr (KIND == kUpper || KIND == kLower) {
         if (a.bt_m && wide && lut && !R64)
-            k_search<KIND, U, true, true, SK, false, 0, true><<<blocks, kBtThreads, lds, s>>>(keys, a);
+            k_search<KIND, U, true, true, SK, false, false, true><<<blocks, kBtThreads, lds, s>>>(keys, a);
         else if (a.bt_m && lut && !R64)
-            k_search<KIND, U, false, true, SK, false, 0, true><<<blocks, kBtThreads, lds, s>>>(keys, a);
+            k_search<KIND, U, false, true, SK, false, false, true><<<blocks, kBtThreads, lds, s>>>(keys, a);
         else if (wide && lut) k_search<KIND, U, true, true, SK, R64><<<blocks, 256, lds, s>>>(keys, a);
         else if (wide) k_search<KIND, U, true, false, SK, R64><<<blocks, 256, 0, s>>>(keys, a);
         else if (lut) k_search<KIND, U, false, true, SK, R64><<<blocks, 256, lds, s>>>(keys, a);
         else k_search<KIND, U, false, false, SK, R64><<<blocks, 256, 0, s>>>(keys, a);
     } else if constexpr (KIND == kLeafRot) {
-        const size_t canon_lds = ((size_t)2) << a.leaf;  // least-rotation table, leaves of <= kNecklaceMax keys
-        if (a.bt_m && !R64 && a.leaf <= kNecklaceMax)
-            k_search<KIND, U, false, false, SK, false, 2, true><<<blocks, kBtThreadsLeaf, canon_lds, s>>>(keys, a);
-        else if (a.bt_m && !R64 && a.leaf <= 16)
-            k_search<KIND, U, false, false, SK, false, 1, true><<<blocks, kBtThreadsLeaf, 0, s>>>(keys, a);
+        const size_t canon_lds = a.leaf <= kNecklaceMax ? ((size_t)2) << a.leaf : 0;  // least-rotation table
+        if (a.leaf >= kStagedMinLeaf)
+            k_search<KIND, U, false, false, true, R64, true><<<blocks, 256, canon_lds, s>>>(keys, a);
         else if (a.bt_m && !R64)
-            k_search<KIND, U, false, false, SK, false, 0, true><<<blocks, kBtThreadsLeaf, 0, s>>>(keys, a);
-        else if (a.leaf <= kNecklaceMax)
-            k_search<KIND, U, false, false, SK, R64, 2><<<blocks, 256, canon_lds, s>>>(keys, a);
-        else if (a.leaf <= 16)
-            k_search<KIND, U, false, false, SK, R64, 1><<<blocks, 256, 0, s>>>(keys, a);
+            k_search<KIND, U, false, false, SK, false, false, true><<<blocks, kBtThreadsLeaf, canon_lds, s>>>(keys, a);
         else
-            k_search<KIND, U, false, false, SK, R64><<<blocks, 256, 0, s>>>(keys, a);
+            k_search<KIND, U, false, false, SK, R64><<<blocks, 256, canon_lds, s>>>(keys, a);
+    } else if constexpr (KIND == kLeafBrute) {
+        k_search<KIND, U, false, false, true, R64, true><<<blocks, 256, 0, s>>>(keys, a);
     } else {
         k_search<KIND, U, false, false, SK, R64><<<blocks, 256, 0, s>>>(keys, a);
     }
@@ -556,9 +552,9 @@ struct SearchShape {
     bool bt;
 };
 static SearchShape search_shape(const Tune &tn, uint32_t kind, bool wide, bool lut, bool r64, bool mostly_full,
-                                uint32_t blocks4, uint32_t full_blocks4, uint32_t num_cus) {
+                                uint32_t blocks4, uint32_t full_blocks4, uint32_t num_cus, uint32_t leaf_size) {
     const bool aggr = tn.bt && (kind == kUpper || kind == kLower) && lut && (!wide || tn.bt_wide) && mostly_full;
-    const bool leaf = tn.bt_leaf && kind == kLeafRot;
+    const bool leaf = tn.bt_leaf && kind == kLeafRot && leaf_size < kStagedMinLeaf;
     const uint32_t wpg = bt_threads((int)kind) / 64;  // waves per workgroup
     // A leaf level of fewer waves than half a byte-table workgroup per CU would
     // put its waves on a few CUs (sharing their SIMDs) while others idle; it runs
@@ -840,7 +836,7 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
             if (!lut) lds = 0;
         }
         const SearchShape sh =
-            search_shape(tn, kind, wide, lut, r64, 2 * cen.full[l] >= cnt, lblocks, blocks, (uint32_t)c->num_cus);
+            search_shape(tn, kind, wide, lut, r64, 2 * cen.full[l] >= cnt, lblocks, blocks, (uint32_t)c->num_cus, leaf);
         a.bt_m = sh.bt ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
         a.n_waves = sh.waves;
         if (sh.waves > n_waves) throw BuildError(RS_ERR_INTERNAL, "search launch beyond the running table");

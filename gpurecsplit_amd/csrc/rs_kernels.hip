@@ -639,8 +639,6 @@ constexpr uint32_t kBtThreads = RS_BT_THREADS;
 #ifndef RS_BT_THREADS_LEAF
 #define RS_BT_THREADS_LEAF 768
 #endif
-// the rotation-leaf instances: 768 as well (512, four waves per SIMD without the
-// spills of the 80-register bound, measured slower: C3 leaves 319 -> 351 ms)
 constexpr uint32_t kBtThreadsLeaf = RS_BT_THREADS_LEAF;
 __host__ __device__ constexpr uint32_t bt_threads(int kind) { return kind == kLeafRot ? kBtThreadsLeaf : kBtThreads; }
 
@@ -680,142 +678,57 @@ constexpr uint32_t kNecklaceMax = 12;
 // seed j*L; keys with even `second` set bits of the left mask, odd ones of the
 // right mask; the lowest r with left | rotl(right, r) == 2^L-1 gives seed j*L+r.
 // The partition places a full leaf's even keys first: kp[0, nl) even, kp[nl, L) odd.
-template <int U, bool SK, bool R64, int RB, bool BT = false>
+// This single pass serves the leaves below kStagedMinLeaf keys (staged leaves below
+// hash most candidates' keys only in part).  Both masks share one word, the left
+// one in bits 0..L-1 and the right one in bits 16..16+L-1.  canon[x] is the least
+// rotation of the L-bit mask x: some rotation of the right mask equals the left
+// mask's complement exactly when both have the same least rotation (which also
+// makes both halves collision-free: a collision changes a popcount), so a candidate
+// costs one pair of table reads; the first match in unit order then finds its
+// lowest fitting rotation across the wave (lane r tests rotation r).
+template <int U, bool SK, bool R64, bool BT>
 __device__ __forceinline__ uint64_t group_leaf_rot(const uint64_t *__restrict__ kp, uint32_t L, uint32_t nl,
-                                                   uint32_t nr, uint64_t u0, const uint16_t *canon) {
+                                                   uint64_t u0, const uint16_t *canon) {
     // BT: position (h16 * L) >> 16 of every 16-bit hash read from the byte table
     const uint8_t *bt = bt_table<BT>();
     const uint64_t S = c_start_seed[kSeedLeaf];
     const uint32_t full = (uint32_t)((1ull << L) - 1);
     const Seeds<U> sd(u0 * L + S, L);
     const uint32_t lane = lane_id();
-    if constexpr (!RB) {
-        // Leaves of 17 to 24 keys: two masks per candidate.  Few candidates per
-        // group are collision-free (1.6 of 256 at L = 18); they are tested in index
-        // order one at a time across the wave: lane r tests rotation r.
-        uint32_t ml[U], mr[U];
+    uint32_t mk[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) ml[u] = mr[u] = 0;
-        if constexpr (R64) {
-            each_r64<U>(kp, 0, nl, sd, L, [&](int u, uint32_t r) { ml[u] |= 1u << r; });
-            each_r64<U>(kp, nl, L, sd, L, [&](int u, uint32_t r) { mr[u] |= 1u << r; });
-        } else if constexpr (BT) {
-            each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { ml[u] |= 1u << bt[h]; });
-            each_hash<U, SK>(kp, nl, L, sd, [&](int u, uint32_t h) { mr[u] |= 1u << bt[h]; });
-        } else {
-            each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { ml[u] |= 1u << (__umul24(h, L) >> 16); });
-            each_hash<U, SK>(kp, nl, L, sd, [&](int u, uint32_t h) { mr[u] |= 1u << (__umul24(h, L) >> 16); });
-        }
-        const uint32_t r = lane < L ? lane : 0;
+    for (int u = 0; u < U; u++) mk[u] = 0;
+    if constexpr (R64) {
+        each_r64<U>(kp, 0, nl, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
+        each_r64<U>(kp, nl, L, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << (r + 16); });
+    } else if constexpr (BT) {
+        uint32_t mr[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            unsigned long long cand = __ballot((uint32_t)__popc(ml[u]) == nl && (uint32_t)__popc(mr[u]) == nr);
-            while (cand) {
-                const int l = __ffsll((long long)cand) - 1;
-                cand &= cand - 1;
-                const uint32_t bl = (uint32_t)__builtin_amdgcn_readlane((int)ml[u], l);
-                const uint32_t br = (uint32_t)__builtin_amdgcn_readlane((int)mr[u], l);
-                const uint32_t rot = r == 0 ? br : (((br << r) | (br >> (L - r))) & full);
-                const unsigned long long fit = __ballot(lane < L && (bl | rot) == full);
-                if (fit) return (u0 + (uint64_t)(u * 64 + l)) * L + (uint64_t)(__ffsll((long long)fit) - 1);
-            }
-        }
-        return kNone;
+        for (int u = 0; u < U; u++) mr[u] = 0;
+        each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { mk[u] |= 1u << bt[h]; });
+        each_hash<U, SK>(kp, nl, L, sd, [&](int u, uint32_t h) { mr[u] |= 1u << bt[h]; });
+#pragma unroll
+        for (int u = 0; u < U; u++) mk[u] |= mr[u] << 16;
     } else {
-        // Leaves of at most 16 keys (RB): both masks in one word, the left one in
-        // bits 0..L-1 and the right one in bits 16..16+L-1 (the 16 folds into the
-        // remap's multiply-add); both halves are collision-free exactly when L bits
-        // are set.  Many candidates pass (13 of 256 at L = 12, 43 at L = 8): they go
-        // to a per-wave LDS list in unit order (u, then lane), and each step tests
-        // floor(64 / L) of them: lane i tests rotation i mod L of candidate i / L,
-        // so the lowest set bit of the ballot is the lowest fitting rotation of the
-        // first candidate that has one.
-        uint32_t mk[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) mk[u] = 0;
-        if constexpr (R64) {
-            each_r64<U>(kp, 0, nl, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
-            each_r64<U>(kp, nl, L, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << (r + 16); });
-        } else if constexpr (BT) {
-            uint32_t mr[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) mr[u] = 0;
-            each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { mk[u] |= 1u << bt[h]; });
-            each_hash<U, SK>(kp, nl, L, sd, [&](int u, uint32_t h) { mr[u] |= 1u << bt[h]; });
-#pragma unroll
-            for (int u = 0; u < U; u++) mk[u] |= mr[u] << 16;
-        } else {
-            each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { mk[u] |= 1u << (__umul24(h, L) >> 16); });
-            each_hash<U, SK>(kp, nl, L, sd,
-                             [&](int u, uint32_t h) { mk[u] |= 1u << ((__umul24(h, L) + (16u << 16)) >> 16); });
-        }
-        if constexpr (RB == 2) {
-            // Leaves of at most kNecklaceMax keys: canon[x] is the least rotation of
-            // the L-bit mask x.  Some rotation of the right mask equals the left
-            // mask's complement exactly when both have the same least rotation
-            // (which also makes both halves collision-free: a collision changes a
-            // popcount), so one pair of table reads per candidate replaces the list
-            // and its steps; the first matching candidate in unit order then finds
-            // its lowest fitting rotation across the wave (lane r tests rotation r).
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool match = canon[mk[u] >> 16] == canon[~mk[u] & full];
-                const unsigned long long bal = __ballot(match);
-                if (bal) {
-                    const int l = __ffsll((long long)bal) - 1;
-                    const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)mk[u], l);
-                    const uint32_t bl = e & 0xFFFFu, br = e >> 16;
-                    const uint32_t r = lane < L ? lane : 0;
-                    const uint32_t rot = r == 0 ? br : (((br << r) | (br >> (L - r))) & full);
-                    const unsigned long long fit = __ballot(lane < L && (bl | rot) == full);
-                    return (u0 + (uint64_t)(u * 64 + l)) * L + (uint64_t)(__ffsll((long long)fit) - 1);
-                }
-            }
-            return kNone;
-        }
-        // one list per wave of the workgroup: masks, and unit indexes (< 256) as bytes
-        constexpr int kWaves = (BT ? kBtThreadsLeaf : 256) / 64;
-        __shared__ uint32_t s_cand_m[kWaves][U * 64];
-        __shared__ uint8_t s_cand_u[kWaves][U * 64];
-        uint32_t *cm = s_cand_m[threadIdx.x >> 6];
-        uint8_t *cu = s_cand_u[threadIdx.x >> 6];
-        uint32_t count = 0;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const bool ok = (uint32_t)__popc(mk[u]) == L;
-            const unsigned long long bal = __ballot(ok);
-            const uint32_t below =
-                __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-            if (ok) {
-                cm[count + below] = mk[u];
-                cu[count + below] = (uint8_t)(u * 64 + lane);
-            }
-            count += (uint32_t)__popcll(bal);
-        }
-        if (count == 0) return kNone;
-        // the list is read back by other lanes of this wave: wait for the writes
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const uint32_t per_step = 64 / L;
-        const uint32_t g = (lane * ((65536 + L - 1) / L)) >> 16;  // lane / L (lane < 64, L <= 16)
-        const uint32_t r = lane - g * L;
-        for (uint32_t base = 0; base < count; base += per_step) {
-            const uint32_t idx = base + g;
-            const bool valid = g < per_step && idx < count;
-            const uint32_t e = valid ? cm[idx] : 0;
-            const uint32_t bl = e & 0xFFFFu, br = e >> 16;
-            const uint32_t rot = r == 0 ? br : (((br << r) | (br >> (L - r))) & full);
-            const unsigned long long fit = __ballot(valid && (bl | rot) == full);
-            if (fit) {
-                const uint32_t first = (uint32_t)__ffsll((long long)fit) - 1;
-                const uint32_t gi = first / L;
-                const uint32_t unit = cu[base + gi];
-                return (u0 + (uint64_t)unit) * L + (uint64_t)(first - gi * L);
-            }
-        }
-        return kNone;
+        each_hash<U, SK>(kp, 0, nl, sd, [&](int u, uint32_t h) { mk[u] |= 1u << (__umul24(h, L) >> 16); });
+        each_hash<U, SK>(kp, nl, L, sd,
+                         [&](int u, uint32_t h) { mk[u] |= 1u << ((__umul24(h, L) + (16u << 16)) >> 16); });
     }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const bool match = canon[mk[u] >> 16] == canon[~mk[u] & full];
+        const unsigned long long bal = __ballot(match);
+        if (bal) {
+            const int l = __ffsll((long long)bal) - 1;
+            const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)mk[u], l);
+            const uint32_t bl = e & 0xFFFFu, br = e >> 16;
+            const uint32_t r = lane < L ? lane : 0;
+            const uint32_t rot = r == 0 ? br : (((br << r) | (br >> (L - r))) & full);
+            const unsigned long long fit = __ballot(lane < L && (bl | rot) == full);
+            return (u0 + (uint64_t)(u * 64 + l)) * L + (uint64_t)(__ffsll((long long)fit) - 1);
+        }
+    }
+    return kNone;
 }
 
 // Leaf without rotation (SIMDRecSplit.hpp:510-599): lowest x whose m keys land on
@@ -850,22 +763,311 @@ __device__ __forceinline__ uint64_t group_leaf_brute(const uint64_t *__restrict_
     return kNone;
 }
 
+// ------------------------------------------------------------------ staged leaves
+
+// Leaves reject most candidates early: a candidate dies at the first two keys that
+// share a position, and of the candidates of an 18-key leaf 16% survive 8 keys.
+// The staged search hashes a prefix of the keys for every candidate, packs the
+// survivors of a wave into an LDS queue (in candidate order) and hashes the other
+// keys for full waves of survivors only.  Expected keys hashed per candidate:
+// 8 + 0.16 * 10 = 9.6 of 18, 10 + 0.11 * 14 = 11.6 of 24, 8 + 0.12 * 8 = 9 of 16.
+// Leaves below kStagedMinLeaf keys take the single pass: their prefix keeps too
+// many candidates, and their whole search is only a few groups.
+constexpr uint32_t kStagedMinLeaf = 12;
+constexpr uint32_t kStagedFill = 48;       // queued candidates that start a second stage
+constexpr uint32_t kStagedCap = 64 + 256;  // queue entries per wave: a rest of < 64, then one group's survivors
+
+// Keys of the first stage for a leaf of m keys: the k that minimises
+// k + 1.4 P(k) (m - k), P(k) the chance that k keys meet no collision (a survivor's
+// key costs about 1.4 of a first-stage key).  Rotation leaves take them from the
+// larger parity half, which has at least ceil(m / 2) >= k keys for every m.
+__host__ __device__ constexpr uint32_t stage_keys(uint32_t m) {
+    double best = 1e9;
+    uint32_t arg = m;
+    double p = 1;
+    for (uint32_t k = 1; k <= (m + 1) / 2; k++) {
+        p *= (double)(m - k + 1) / (double)m;
+        const double c = (double)k + 1.4 * p * (double)(m - k);
+        if (c < best) {
+            best = c;
+            arg = k;
+        }
+    }
+    return arg;
+}
+struct StageTable {
+    uint8_t k[kMaxLeaf + 1];
+    constexpr StageTable() : k{} {
+        for (uint32_t m = 2; m <= kMaxLeaf; m++) k[m] = (uint8_t)stage_keys(m);
+    }
+};
+__constant__ StageTable c_stage = StageTable();
+
+// Position floor(h16 * m / 2^16) of a 16-bit hash; m16 = m << 16 (24-bit operands).
+__device__ __forceinline__ uint32_t pos_of(uint32_t h, uint32_t m16) {
+    uint32_t r;
+    __asm__("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(r) : "s"(m16), "v"(h));
+    return r;
+}
+
+// pos_of(h16_of(hash_post16(t)), m16) as one block.  The s_nop after the shift lets
+// the scheduler issue another wave's full-rate instruction beside this one's (31.5
+// cycles per key and SIMD against 33.8 without it, 40.6 with no break in the chain);
+// the one after the word-select xor is the wait its reader needs.
+__device__ __forceinline__ uint32_t post_pos(uint32_t t, uint32_t m16) {
+    uint32_t x;
+    __asm__("v_mul_lo_u32 %0, %0, %2\n\t"
+            "v_lshrrev_b32 %1, 13, %0\n\t"
+            "s_nop 0\n\t"
+            "v_xor_b32 %0, %0, %1\n\t"
+            "v_mul_lo_u32 %0, %0, %3\n\t"
+            "v_xor_b32_sdwa %0, %0, %0 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+            "s_nop 0\n\t"
+            "v_mul_hi_u32_u24 %0, %4, %0"
+            : "+v"(t), "=&v"(x)
+            : "s"(0x85ebca6bu), "s"(0xc2b2ae35u), "s"(m16));
+    return t;
+}
+
+// Calls g(pos) for every key of kp[begin, end) and this lane's own candidate at
+// base + off (off < 2^32, at most max_off over the wave).
+template <bool R64, typename G>
+__device__ __forceinline__ void each_pos_lane(const uint64_t *__restrict__ kp, uint32_t begin, uint32_t end,
+                                              uint64_t base_any, uint32_t off, uint32_t max_off, uint32_t m, G &&g) {
+    const uint64_t base = uni64(base_any);
+    if constexpr (R64) {
+        stream_keys_scalar(kp, begin, end, [&](uint64_t k) { g(remap64(k + base + off, m)); });
+    } else {
+        const uint32_t m16 = uni(m << 16), mo = uni(max_off);
+        stream_keys_scalar(kp, begin, end, [&](uint64_t k) {
+            const uint64_t S = k + base;
+            const uint32_t lo = (uint32_t)S, hi = (uint32_t)(S >> 32);
+            if (lo <= ~mo) g(pos_of(h16_of(hash_pre32((lo + off) ^ hi)), m16));
+            else g(pos_of(search_h16(S + off), m16));
+        });
+    }
+}
+
+// Per-wave state of a staged search: the survivors' queue in LDS and its fill.
+struct StageQueue {
+    uint2 *q;      // {position mask, candidate index relative to the claim's first}
+    uint32_t n;    // entries (wave-uniform)
+};
+
+__device__ __forceinline__ uint2 *stage_queue() {
+    __shared__ uint2 s_stage[4][kStagedCap];
+    return s_stage[threadIdx.x >> 6];
+}
+
+// Keys of the first stage, in scalar registers for a whole claim (their loads and
+// waits leave the group loop): kStageKeys covers stage_keys(m) of every m <= 24.
+constexpr int kStageKeys = 12;
+struct StageKeys {
+    uint64_t k[kStageKeys];
+    uint32_t n;
+    // kp[0, 12) is readable: a staged node has at least 12 keys, its stage starts no
+    // later than key m / 2, and the key array carries 8 entries of padding
+    __device__ __forceinline__ void load(const uint64_t *kp_any, uint32_t n_any) {
+        typedef unsigned int u32x8 __attribute__((ext_vector_type(8)));
+        const uint64_t *kp = (const uint64_t *)uni64((uint64_t)kp_any);
+        n = uni(n_any);
+        uint64_t lo[8];
+        sload_keys8(kp, lo);
+        u32x8 r;
+        __asm__ volatile("s_load_dwordx8 %0, %1, 0x40\n\ts_waitcnt lgkmcnt(0)" : "=&s"(r) : "s"(kp) : "memory");
+#pragma unroll
+        for (int j = 0; j < 8; j++) k[j] = lo[j];
+#pragma unroll
+        for (int j = 0; j < 4; j++) k[8 + j] = ((uint64_t)r[2 * j + 1] << 32) | r[2 * j];
+    }
+};
+
+// First stage of one group: candidates idx0 + u * 64 + lane, u < U, of the claim
+// that starts at absolute base seed `base` (stride apart).
+template <int U, bool R64>
+__device__ __forceinline__ void stage_push(const StageKeys &sk, uint64_t base, uint32_t stride, uint32_t m,
+                                           uint32_t idx0, StageQueue &sq) {
+    const uint32_t lane = lane_id();
+    uint32_t mk[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) mk[u] = 0;
+    const Seeds<U> sd(base + (uint64_t)idx0 * stride, stride);
+    const uint64_t sb = uni64(sd.base);
+    const uint32_t m16 = uni(m << 16), max_off = uni(sd.max_off);
+#pragma unroll
+    for (int j = 0; j < kStageKeys; j++) {
+        if ((uint32_t)j >= sk.n) continue;
+        const uint64_t S = sk.k[j] + sb;
+        if constexpr (R64) {
+#pragma unroll
+            for (int u = 0; u < U; u++) mk[u] |= 1u << remap64(S + sd.off[u], m);
+        } else {
+            // as each_hash: one add and one xor per candidate away from a 2^16 boundary
+            const uint32_t lo = (uint32_t)S, hi = (uint32_t)(S >> 32);
+            if ((lo & 0xFFFFu) <= 0xFFFFu - max_off) {
+                const uint32_t D = hi ^ (hi >> 16) ^ (lo >> 16);
+#pragma unroll
+                for (int u = 0; u < U; u++) mk[u] |= 1u << post_pos((lo + sd.off[u]) ^ D, m16);
+            } else if (lo <= ~max_off) {
+#pragma unroll
+                for (int u = 0; u < U; u++) mk[u] |= 1u << pos_of(h16_of(hash_pre32((lo + sd.off[u]) ^ hi)), m16);
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; u++) mk[u] |= 1u << pos_of(search_h16(S + sd.off[u]), m16);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const bool ok = (uint32_t)__popc(mk[u]) == sk.n;
+        const unsigned long long bal = __ballot(ok);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+        if (ok) sq.q[sq.n + below] = make_uint2(mk[u], idx0 + u * 64 + lane);
+        sq.n = uni(sq.n + (uint32_t)__popcll(bal));
+    }
+    // the queue is read back by other lanes of this wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Lowest fitting rotation of the first lane (in lane order) of `cand` whose masks
+// ml (even keys) and mr (odd keys) of L bits fit: lane * L + rotation, or kNone.
+// Lane i tests rotation i mod L of candidate i / L, floor(64 / L) candidates per step.
+__device__ __forceinline__ uint64_t fit_rotation(unsigned long long cand, uint32_t ml, uint32_t mr, uint32_t L) {
+    const uint32_t lane = lane_id(), full = (uint32_t)((1ull << L) - 1);
+    const uint32_t r = lane < L ? lane : 0;
+    while (cand) {
+        const int l = __ffsll((long long)cand) - 1;
+        cand &= cand - 1;
+        const uint32_t bl = (uint32_t)__builtin_amdgcn_readlane((int)ml, l);
+        const uint32_t br = (uint32_t)__builtin_amdgcn_readlane((int)mr, l);
+        const uint32_t rot = r == 0 ? br : (((br << r) | (br >> (L - r))) & full);
+        const unsigned long long fit = __ballot(lane < L && (bl | rot) == full);
+        if (fit) return (uint64_t)l * L + (uint64_t)(__ffsll((long long)fit) - 1);
+    }
+    return kNone;
+}
+
+// Second stage of the first min(64, n) queued candidates: hashes their remaining
+// keys and tests them; moves the queue's rest to its front.  Returns the lowest
+// valid seed relative to the claim (candidate index, times L plus the rotation for
+// rotation leaves) or kNone.  Rotation leaves: kp[0, nl) even, kp[nl, L) odd; the
+// first stage took the first k keys of the larger half.
+template <bool ROT, bool R64>
+__device__ __forceinline__ uint64_t stage_test(const uint64_t *__restrict__ kp, uint32_t m, uint32_t nl, uint32_t k,
+                                               uint64_t base, uint32_t stride, uint32_t max_idx, StageQueue &sq,
+                                               const uint16_t *canon) {
+    const uint32_t lane = lane_id();
+    const uint32_t cnt = sq.n < 64 ? sq.n : 64;
+    const uint2 e = sq.q[lane < cnt ? lane : 0];
+    const bool valid = lane < cnt;
+    const uint32_t off = e.y * stride, max_off = max_idx * stride;
+    const uint32_t full = (uint32_t)((1ull << m) - 1);
+    uint64_t hit = kNone;
+    if constexpr (!ROT) {
+        uint32_t mk = e.x;
+        each_pos_lane<R64>(kp, k, m, base, off, max_off, m, [&](uint32_t r) { mk |= 1u << r; });
+        const unsigned long long bal = __ballot(valid && mk == full);
+        if (bal) hit = (uint32_t)__builtin_amdgcn_readlane((int)e.y, __ffsll((long long)bal) - 1);
+    } else {
+        const bool even_first = 2 * nl >= m;
+        const uint32_t b1 = even_first ? k : nl + k, e1 = even_first ? nl : m;  // rest of the larger half
+        const uint32_t b2 = even_first ? nl : 0, e2 = even_first ? m : nl;      // the other half
+        uint32_t m1 = e.x, m2 = 0;
+        each_pos_lane<R64>(kp, b1, e1, base, off, max_off, m, [&](uint32_t r) { m1 |= 1u << r; });
+        each_pos_lane<R64>(kp, b2, e2, base, off, max_off, m, [&](uint32_t r) { m2 |= 1u << r; });
+        const uint32_t ml = even_first ? m1 : m2, mr = even_first ? m2 : m1;
+        unsigned long long cand;
+        // canon (leaves of at most kNecklaceMax keys): the least rotations decide,
+        // and only the first matching candidate looks for its rotation
+        if (m <= kNecklaceMax) {
+            cand = __ballot(valid && canon[mr] == canon[~ml & full]);
+            cand &= 0 - cand;
+        } else {
+            cand = __ballot(valid && (uint32_t)__popc(ml) == nl && (uint32_t)__popc(mr) == m - nl);
+        }
+        const uint64_t f = fit_rotation(cand, ml, mr, m);
+        if (f != kNone) {
+            const uint32_t l = (uint32_t)f / m;
+            hit = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)e.y, (int)l) * m + ((uint32_t)f - l * m);
+        }
+    }
+    const uint32_t left = sq.n - cnt;
+    for (uint32_t i = lane; i < left; i += 64) {
+        // entry 64 + i moves to i; i + 64 is read before any lane of a later
+        // iteration writes it, and iterations run in increasing order
+        const uint2 t = sq.q[64 + i];
+        __builtin_amdgcn_wave_barrier();
+        sq.q[i] = t;
+    }
+    sq.n = left;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return hit;
+}
+
+// One claim of a staged leaf search: n_groups groups of U * 64 candidates from unit0
+// on, stopped by a lower result of another wave (*result, in seeds: unit * scale).
+// Returns the lowest valid seed or kNone; *work counts the key evaluations.  A
+// function of its own: inlined, the claim loop's values crowd the stage's keys out
+// of the scalar registers (C3 rotation leaves 233 -> 302 ms by spills into lanes).
+template <bool ROT, int U, bool R64>
+__device__ __noinline__ uint64_t staged_claim(const uint64_t *kp_any, uint32_t m_any, uint32_t nl_any, uint64_t unit0_any,
+                                              uint32_t n_groups_any, const unsigned long long *result_any,
+                                              const uint16_t *canon, uint32_t *groups_run, uint32_t *tests_run) {
+    const uint64_t *kp = (const uint64_t *)uni64((uint64_t)kp_any);
+    const unsigned long long *result = (const unsigned long long *)uni64((uint64_t)result_any);
+    const uint32_t m = uni(m_any), nl = uni(nl_any), n_groups = uni(n_groups_any);
+    const uint64_t unit0 = uni64(unit0_any);
+    const uint32_t stride = ROT ? m : 1;
+    const uint64_t base = unit0 * stride + c_start_seed[kSeedLeaf];
+    const uint32_t k = uni(c_stage.k[m]), max_idx = n_groups * U * 64 - 1;
+    const uint32_t b = ROT && 2 * nl < m ? nl : 0;  // the larger half's first key
+    StageQueue sq{stage_queue(), 0};
+    StageKeys sk;
+    sk.load(kp + b, k);
+    uint64_t hit = kNone;
+    uint32_t g = 0, tests = 0;
+    while (g < n_groups && hit == kNone) {
+        if (g > 0) {
+            unsigned long long r = 0;
+            if (lane_id() == 0) r = ld_relaxed(result);
+            r = uni64(r);
+            if ((unit0 + (uint64_t)g * U * 64) * stride >= r) break;
+        }
+        stage_push<U, R64>(sk, base, stride, m, g * U * 64, sq);
+        g++;
+        while (sq.n >= kStagedFill && hit == kNone) {
+            hit = stage_test<ROT, R64>(kp, m, nl, k, base, stride, max_idx, sq, canon);
+            tests++;
+        }
+    }
+    // the queue is drained before the claim ends, so its entries never outlive a node
+    while (sq.n && hit == kNone) {
+        hit = stage_test<ROT, R64>(kp, m, nl, k, base, stride, max_idx, sq, canon);
+        tests++;
+    }
+    *groups_run = g;
+    *tests_run = tests;
+    return hit == kNone ? kNone : hit + unit0 * stride;
+}
+
 __device__ __forceinline__ bool has_work(const NodeState *st, uint64_t units_per_chunk, uint64_t scale) {
     const unsigned long long nc = ld_relaxed(&st->next_chunk);
     const unsigned long long res = ld_relaxed(&st->result);
     return nc * units_per_chunk * scale < res;
 }
 
-// RB (rotation leaves of at most 16 keys): packed masks, and the candidate test
-// batched through LDS (RB = 1) or, for at most kNecklaceMax keys, through the
-// table of least rotations (RB = 2), with registers held to five waves per SIMD.  BT
-// (aggregation levels, 32-bit counters, 16-bit remap): the byte table for nodes of
-// bt_m keys, workgroups of kBtThreads threads, two per CU (registers held to the
-// kBtThreads / 128 waves per SIMD that two such workgroups need).
-template <int KIND, int U, bool WIDE, bool LUT, bool SK, bool R64, int RB = 0, bool BT = false>
-__global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) / 128 : (RB ? 5 : 1)) void k_search(const uint64_t *__restrict__ keys,
+// ST (leaf kinds): leaves of at least kStagedMinLeaf keys run the staged search.  BT
+// (aggregation levels and rotation leaves below kStagedMinLeaf, 16-bit remap): the
+// byte table for nodes of bt_m keys, workgroups of kBtThreads threads, two per CU
+// (registers held to the kBtThreads / 128 waves per SIMD that two such workgroups need).
+template <int KIND, int U, bool WIDE, bool LUT, bool SK, bool R64, bool ST = false, bool BT = false>
+__global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) / 128 : (KIND == kLeafRot ? 5 : 1)) void k_search(const uint64_t *__restrict__ keys,
                                                                                   SearchArgs a) {
-    static_assert(!BT || ((((KIND == kUpper || KIND == kLower) && LUT && !RB) || KIND == kLeafRot) && !R64),
+    static_assert(!BT || ((((KIND == kUpper || KIND == kLower) && LUT) || KIND == kLeafRot) && !R64 && !ST),
                   "the byte table serves aggregation levels and rotation leaves over the 16-bit remap");
     extern __shared__ uint32_t s_lut[];
     const uint32_t lane = lane_id();
@@ -917,7 +1119,7 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
         }
         __syncthreads();
     }
-    if constexpr (KIND == kLeafRot && RB == 2) {
+    if (KIND == kLeafRot && (!ST || a.leaf <= kNecklaceMax)) {
         // least rotation of every L-bit mask, in the dynamic LDS (2^L entries)
         uint16_t *canon = (uint16_t *)s_lut;
         const uint32_t L = a.leaf, full = (1u << L) - 1;
@@ -1054,7 +1256,6 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
                 const bool odd_key = lane < m && (keys[key_off + lane] & 1) != 0;
                 const uint32_t odd = (uint32_t)__popcll(__ballot(odd_key));
                 aux0 = m - odd;  // nl
-                aux1 = odd;      // nr
             } else {
                 uint32_t mid = m;
                 if (m >= 14) {
@@ -1113,7 +1314,17 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
         }
         const uint64_t *kp = keys + key_off;
         uint64_t hit = kNone;
-        for (uint32_t g = 0; g < a.groups * span; g++) {
+        if constexpr (ST) {
+            if (KIND == kLeafRot || m >= kStagedMinLeaf) {
+                uint32_t groups_run, tests_run;
+                hit = staged_claim<KIND == kLeafRot, U, R64>(kp, m, aux0, unit0, a.groups * span, &a.state[node].result,
+                                                             (const uint16_t *)s_lut, &groups_run, &tests_run);
+                const uint32_t k = c_stage.k[m];
+                work += (uint64_t)groups_run * U * 64 * k + (uint64_t)tests_run * 64 * (m - k);
+            }
+        }
+        const bool single = !ST || (KIND == kLeafBrute && m < kStagedMinLeaf);
+        for (uint32_t g = 0; single && g < a.groups * span; g++) {
             const uint64_t u0 = unit0 + (uint64_t)g * U * 64;
             if (g > 0) {
                 unsigned long long r = 0;
@@ -1128,8 +1339,8 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
             else if (KIND == kUpper || KIND == kLower)
                 hit = group_aggr<U, WIDE, LUT, SK, R64>(kp, m, sconst, a.field_bits, a.magic, T, cmask, lut_hi, two,
                                                         u0);
-            else if (KIND == kLeafRot)
-                hit = group_leaf_rot<U, SK, R64, RB, BT>(kp, m, aux0, aux1, u0, (const uint16_t *)s_lut);
+            else if (KIND == kLeafRot && !ST)
+                hit = group_leaf_rot<U, SK, R64, BT>(kp, m, aux0, u0, (const uint16_t *)s_lut);
             else hit = group_leaf_brute<U, SK, R64>(kp, m, aux0, u0);
             if (hit != kNone) break;
         }

@@ -60,7 +60,8 @@ struct NodeDesc {
 };
 
 // Search state of one node (32 B): lowest valid seed found so far, the next
-// unclaimed chunk of candidate seeds, and the number of waves working on it.
+// unclaimed chunk of candidate seeds, the number of waves working on it, and, for
+// nodes searched packed, their key classes' bounds (12 bits each, pk_bound).
 struct NodeState {
     unsigned long long result;
     unsigned long long next_chunk;

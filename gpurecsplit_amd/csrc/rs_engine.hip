@@ -307,6 +307,7 @@ struct Tune {
     // fanout-2 nodes need ~40 candidates, so extra waves mostly overshoot
     int help_cap[kNumKinds] = {2, 0, 0, 0, 0};
     int blocks_per_cu = 8;
+    int pk = 1;      // packed parts for the full-size nodes of heavy aggregation levels
     int bt = 1;      // byte table for the full-size nodes of aggregation levels
     int u_bt = 4;    // candidates in flight per lane in those launches
     int bt_leaf = 1; // byte table of positions for rotation leaves
@@ -332,6 +333,7 @@ static Tune parse_tune(const char *env, Tune t = Tune()) {
             else if (k.size() == 2 && k[0] == 'u' && k[1] >= '0' && k[1] < '0' + (int)kNumKinds && uv)
                 t.u[k[1] - '0'] = v;
             else if (k == "lut") t.lut = v != 0;
+            else if (k == "pk") t.pk = v != 0;
             else if (k == "bt") t.bt = v != 0;
             else if (k == "ubt" && uv) t.u_bt = v;
             else if (k == "btl") t.bt_leaf = v != 0;
@@ -361,6 +363,7 @@ static std::string format_tune(const Tune &t) {
     for (int k = 0; k < kNumKinds; k++) add("sk" + std::to_string(k), t.sk[k]);
     for (int k = 0; k < kNumKinds; k++) add("h" + std::to_string(k), t.help_cap[k]);
     add("lut", t.lut);
+    add("pk", t.pk);
     add("bt", t.bt);
     add("ubt", t.u_bt);
     add("btl", t.bt_leaf);
@@ -496,7 +499,11 @@ static double ev_ms(rs_ctx *c, int a, int b) {
 template <int KIND, int U, bool SK, bool R64>
 static void launch_kind(hipStream_t s, const uint64_t *keys, const SearchArgs &a, bool wide, bool lut, uint32_t blocks,
                         size_t lds) {
-    if constexpr (KIND == kUpper || KIND == kLower) {
+    if constexpr (U == kPkU) {
+        static_assert(KIND == kUpper || KIND == kLower, "packed parts serve aggregation levels");
+        if (wide) k_search<KIND, U, true, true, true, false, false, false, true><<<blocks, 256, lds, s>>>(keys, a);
+        else k_search<KIND, U, false, true, true, false, false, false, true><<<blocks, 256, lds, s>>>(keys, a);
+    } else if constexpr (KIND == kUpper || KIND == kLower) {
         if (a.bt_m && wide && lut && !R64)
             k_search<KIND, U, true, true, SK, false, false, true><<<blocks, kBtThreads, lds, s>>>(keys, a);
         else if (a.bt_m && lut && !R64)
@@ -542,6 +549,10 @@ static void launch_sk(hipStream_t s, int u, uint32_t kind, const uint64_t *keys,
     }
 }
 
+// Packed parts (full-size aggregation nodes) from this Golomb-Rice parameter of the
+// level's full size on: 2.08 * 2^12 = 8,500 expected candidates, sixteen groups of 512.
+constexpr uint32_t kPkMinGolomb = 12;
+
 // Grid of one search level from its size in 4-wave workgroups: the byte-table
 // instance (aggregation levels with 32-bit counters whose nodes are mostly of the
 // full size, and rotation leaves, both over the 16-bit remap) runs
@@ -549,10 +560,20 @@ static void launch_sk(hipStream_t s, int u, uint32_t kind, const uint64_t *keys,
 // workgroup.
 struct SearchShape {
     uint32_t grid, waves;
-    bool bt;
+    bool bt, pk;
 };
 static SearchShape search_shape(const Tune &tn, uint32_t kind, bool wide, bool lut, bool r64, bool mostly_full,
-                                uint32_t blocks4, uint32_t full_blocks4, uint32_t num_cus, uint32_t leaf_size) {
+                                uint32_t blocks4, uint32_t full_blocks4, uint32_t num_cus, uint32_t leaf_size,
+                                uint32_t golomb, double nodes) {
+    if (tn.pk && (kind == kUpper || kind == kLower) && lut && !r64 && mostly_full && golomb >= kPkMinGolomb) {
+        // eight independent candidates per lane keep a SIMD busy with few waves, and
+        // waves that only help on other waves' nodes cost more than they give: levels
+        // of fewer nodes than the grid has waves run four waves per SIMD (100K keys at
+        // l = 16: lower 10.3 -> 9.2 ms, upper 5.7 -> 5.2; 1M keys: upper 33.7 -> 32.9;
+        // its lower level of 9,100 nodes keeps the grid, 66.4 ms against 71.0)
+        const uint32_t b = nodes < 4.0 * full_blocks4 ? std::min(blocks4, 4 * num_cus) : blocks4;
+        return {b, b * 4, false, true};
+    }
     const bool aggr = tn.bt && (kind == kUpper || kind == kLower) && lut && (!wide || tn.bt_wide) && mostly_full;
     const bool leaf = tn.bt_leaf && kind == kLeafRot && leaf_size < kStagedMinLeaf;
     const uint32_t wpg = bt_threads((int)kind) / 64;  // waves per workgroup
@@ -564,14 +585,20 @@ static SearchShape search_shape(const Tune &tn, uint32_t kind, bool wide, bool l
     // Small aggregation levels keep the byte table, whose instruction savings
     // outweigh that (10K keys at l = 16: upper 1.68 ms with it, 2.54 ms without).
     const bool fills = (uint64_t)blocks4 * 4 * 2 >= (uint64_t)num_cus * wpg;
-    if (!((aggr || (leaf && fills)) && !r64)) return {blocks4, blocks4 * 4, false};
+    if (!((aggr || (leaf && fills)) && !r64)) return {blocks4, blocks4 * 4, false, false};
     const uint32_t g = std::max<uint32_t>(1, std::min((blocks4 * 4 + wpg - 1) / wpg, full_blocks4 * 4 / wpg));
-    return {g, g * wpg, true};  // never past the full grid
+    return {g, g * wpg, true, false};  // never past the full grid
 }
 
 // The 64-bit remap runs with keys in scalar registers only.
 static void launch_search(hipStream_t s, const Tune &tn, uint32_t kind, const uint64_t *keys, const SearchArgs &a,
-                          bool wide, bool lut, uint32_t blocks, size_t lds, bool r64) {
+                          bool wide, bool lut, uint32_t blocks, size_t lds, bool r64, bool pk) {
+    if (pk) {
+        if (kind == kUpper) launch_kind<kUpper, kPkU, true, false>(s, keys, a, wide, lut, blocks, lds);
+        else launch_kind<kLower, kPkU, true, false>(s, keys, a, wide, lut, blocks, lds);
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     const int u = a.bt_m && (kind == kUpper || kind == kLower) ? (wide ? tn.u_bt_wide : tn.u_bt) : tn.u[kind];
     if (r64) launch_sk<true, true>(s, u, kind, keys, a, wide, lut, blocks, lds);
     else if (tn.sk[kind]) launch_sk<true, false>(s, u, kind, keys, a, wide, lut, blocks, lds);
@@ -802,7 +829,6 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         const uint32_t kind = l < (int)kMaxDepth ? kHigher : (uint32_t)(l - kMaxDepth + 1);
         const NodeDesc *nodes = pool + lbase[l];
         const uint32_t lblocks = level_blocks(cen.evals[l], (double)cnt, blocks);
-        k_state_init<<<(cnt + 255) / 256, 256, 0, s>>>(state, cnt);
         HIP_CHECK(hipMemsetAsync(ctl, 0, 64, s));
         SearchArgs a{};
         a.nodes = nodes;
@@ -836,9 +862,17 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
             if (!lut) lds = 0;
         }
         const SearchShape sh =
-            search_shape(tn, kind, wide, lut, r64, 2 * cen.full[l] >= cnt, lblocks, blocks, (uint32_t)c->num_cus, leaf);
-        a.bt_m = sh.bt ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
+            search_shape(tn, kind, wide, lut, r64, 2 * cen.full[l] >= cnt, lblocks, blocks, (uint32_t)c->num_cus, leaf,
+                         lds ? golomb_param(hmemo, a.lut_entries) : 0, (double)cnt);
+        a.bt_m = sh.bt || sh.pk ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
         a.n_waves = sh.waves;
+        if (sh.pk) {
+            a.groups = 1;
+            k_class_order<<<std::min<uint32_t>(cnt, (uint32_t)c->num_cus * 32), 64, (size_t)a.bt_m * 8, s>>>(
+                sorted, nodes, state, cnt, a.bt_m, kind == kUpper ? kSeedUpper : kSeedLower);
+        } else {
+            k_state_init<<<(cnt + 255) / 256, 256, 0, s>>>(state, cnt);
+        }
         if (sh.waves > n_waves) throw BuildError(RS_ERR_INTERNAL, "search launch beyond the running table");
         HIP_CHECK(hipMemsetAsync(running, 0xFF, (size_t)sh.waves * 4, s));
         st.kind_waves[kind] = std::max(st.kind_waves[kind], sh.waves);
@@ -846,7 +880,7 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         // otherwise be bound by the one fresh-node counter (one atomic per node).
         claim_params(cnt, sh.waves, a.claim_batch, a.batch_tickets);
         PhaseEvents pe{kind, ev_record(c), -1, -1};
-        launch_search(s, tn, kind, sorted, a, wide, lut, sh.grid, lds, r64);
+        launch_search(s, tn, kind, sorted, a, wide, lut, sh.grid, lds, r64, sh.pk);
         pe.search1 = ev_record(c);
         if (kind == kHigher || kind == kUpper || kind == kLower) {
             const uint32_t max_m = kind == kHigher ? st.max_bucket_size : (kind == kUpper ? P.upper : P.lower);

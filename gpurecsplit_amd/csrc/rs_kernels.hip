@@ -670,6 +670,227 @@ __device__ __forceinline__ uint64_t group_aggr_bt(const uint64_t *__restrict__ k
     return kNone;
 }
 
+// ------------------------------------------------------------------ packed parts
+
+// Aggregation nodes of the level's full size m = fan * unit, 16-bit remap (instance
+// PK): part floor(h16 * fan / 2^16) of a key is one 24-bit high multiply, no table.
+//
+// Each lane owns kPkU = 8 consecutive candidates.  With S = key + base (base: the
+// group's first candidate, a multiple of 8 above the level's start seed), the low
+// three bits r of S are the same for every lane and every group of a node, so the
+// keys of a node are ordered once by r (k_class_order) and the code below is
+// instantiated per r.  Candidate u of a lane hashes w = lo(S) + 8 lane + u: slot
+// j = r + u of the aligned block B = lo(S) - r + 8 lane (j < 8) or of B + 8.  Inside
+// an aligned block the fold's xor only permutes the slots, and its first multiply
+// becomes ((B ^ D) + (d ^ j) - d) C = Q + S_j with one vector multiply per block and
+// wave-uniform S_j: two adds, xors and multiplies per key serve eight candidates.
+// The parts of four keys share a register (one byte each), and one dot product adds
+// their squares to the candidate's sum.  A candidate whose counts all equal `unit`
+// has the sum unit * (0 + 1 + 4 + ... + (fan - 1)^2); 0.1 to 0.3% of the others
+// have it too, so every candidate with that sum is counted exactly (lane per key).
+//
+// About 7 vector instructions per evaluation and no LDS, against 8 instructions and
+// one random byte read of a 64 KiB LDS table (the byte-table instance), whose bank
+// conflicts (7.3 LDS cycles per wave read, four SIMDs per LDS) bound it at 30 cycles
+// per evaluation and SIMD: 5M keys at l = 16, b = 2000, lower level 375 -> 330 ms,
+// upper 181 -> 154; 7K keys at l = 24 (no 64-bit counters any more) lower 290 -> 214.
+// A wave instruction takes 3.7 cycles here, so what bounds it is vector issue.
+constexpr int kPkU = 8;
+
+// Part of key + candidate for one slot, into byte Q of x (Q = 0 clears the others):
+// t = q + s is the fold's word after its first multiply (s is zero for slot 0).
+template <int Q, bool ZERO>
+__device__ __forceinline__ void pk_slot(uint32_t &x, uint32_t q, uint32_t s, uint32_t fan16) {
+    uint32_t t, y;
+    if constexpr (ZERO) {
+        __asm__("v_lshrrev_b32 %1, 13, %2\n\t"
+                "v_xor_b32 %0, %2, %1\n\t"
+                "v_mul_lo_u32 %0, %0, %3\n\t"
+                "v_xor_b32_sdwa %0, %0, %0 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+                "s_nop 0"
+                : "=&v"(t), "=&v"(y)
+                : "v"(q), "s"(0xc2b2ae35u));
+    } else {
+        __asm__("v_add_u32 %0, %4, %2\n\t"
+                "v_lshrrev_b32 %1, 13, %0\n\t"
+                "v_xor_b32 %0, %0, %1\n\t"
+                "v_mul_lo_u32 %0, %0, %3\n\t"
+                "v_xor_b32_sdwa %0, %0, %0 dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0\n\t"
+                "s_nop 0"
+                : "=&v"(t), "=&v"(y)
+                : "v"(q), "s"(0xc2b2ae35u), "s"(s));
+    }
+    if constexpr (Q == 0)
+        __asm__("v_mul_hi_u32_u24_sdwa %0, %1, %2 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0"
+                : "=v"(x) : "v"(fan16), "v"(t));
+    else if constexpr (Q == 1)
+        __asm__("v_mul_hi_u32_u24_sdwa %0, %1, %2 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:WORD_0"
+                : "+v"(x) : "v"(fan16), "v"(t));
+    else if constexpr (Q == 2)
+        __asm__("v_mul_hi_u32_u24_sdwa %0, %1, %2 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:WORD_0"
+                : "+v"(x) : "v"(fan16), "v"(t));
+    else
+        __asm__("v_mul_hi_u32_u24_sdwa %0, %1, %2 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:WORD_0"
+                : "+v"(x) : "v"(fan16), "v"(t));
+}
+
+// One key of class R (S mod 8 == R) for the eight candidates, away from a 2^16
+// boundary: (lo mod 2^16) + 8 * 64 + 8 < 2^16.
+template <int R, int Q>
+__device__ __forceinline__ void pk_key(uint64_t S, uint32_t lane8, uint32_t fan16, uint32_t (&x)[kPkU]) {
+    const uint32_t lo = (uint32_t)S, hi = (uint32_t)(S >> 32);
+    const uint32_t D = hi ^ (hi >> 16) ^ (lo >> 16);
+    constexpr uint32_t C = 0x85ebca6bu;
+    const uint32_t b0 = uni(lo - R), b1 = uni(lo - R + 8);  // aligned to 8: lo mod 8 == R
+    const uint32_t q0 = ((b0 + lane8) ^ D) * C;
+    const uint32_t q1 = R ? ((b1 + lane8) ^ D) * C : 0;
+    // slot bit i set adds C << i where bit i of D is clear, subtracts it where it is set
+    const uint32_t s0 = D & 1 ? 0u - C : C, s1 = D & 2 ? 0u - 2 * C : 2 * C, s2 = D & 4 ? 0u - 4 * C : 4 * C;
+    const uint32_t sj[8] = {0, s0, s1, s0 + s1, s2, s2 + s0, s2 + s1, s2 + s1 + s0};
+#define RS_PK_SLOT(u) pk_slot<Q, ((R + u) & 7) == 0>(x[u], R + u < 8 ? q0 : q1, sj[(R + u) & 7], fan16)
+    RS_PK_SLOT(0);
+    RS_PK_SLOT(1);
+    RS_PK_SLOT(2);
+    RS_PK_SLOT(3);
+    RS_PK_SLOT(4);
+    RS_PK_SLOT(5);
+    RS_PK_SLOT(6);
+    RS_PK_SLOT(7);
+#undef RS_PK_SLOT
+}
+
+// Keys kp[b, e) of class R, four per step.
+template <int R>
+__device__ __forceinline__ void pk_class(const uint64_t *kp, uint32_t b, uint32_t e, uint64_t base, uint32_t lane8,
+                                         uint32_t fan16, uint32_t fan, uint32_t (&acc)[kPkU]) {
+    typedef unsigned int u32x8 __attribute__((ext_vector_type(8)));
+    constexpr uint32_t kEdge = 0xFFFFu - (8 * 64 + 8);
+    for (uint32_t i = b; i < e; i += 4) {
+        // kp[i + 3] is readable: the key array carries 8 entries of padding
+        u32x8 r;
+        __asm__ volatile("s_load_dwordx8 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(r) : "s"(kp + i) : "memory");
+        const uint64_t S[4] = {(((uint64_t)r[1] << 32) | r[0]) + base, (((uint64_t)r[3] << 32) | r[2]) + base,
+                               (((uint64_t)r[5] << 32) | r[4]) + base, (((uint64_t)r[7] << 32) | r[6]) + base};
+        const uint32_t rem = e - i;
+        // keys near a 2^16 boundary (0.8%) are hashed in full below
+        uint32_t x[kPkU], edge = 0;
+        if (((uint32_t)S[0] & 0xFFFFu) <= kEdge) {
+            pk_key<R, 0>(S[0], lane8, fan16, x);
+        } else {
+            edge = 1;
+#pragma unroll
+            for (int u = 0; u < kPkU; u++) x[u] = 0;
+        }
+#define RS_PK_KEY(q)                                                                  \
+    if (q < rem) {                                                                    \
+        if (((uint32_t)S[q] & 0xFFFFu) <= kEdge) pk_key<R, q>(S[q], lane8, fan16, x); \
+        else edge |= 1u << q;                                                         \
+    }
+        RS_PK_KEY(1)
+        RS_PK_KEY(2)
+        RS_PK_KEY(3)
+#undef RS_PK_KEY
+#pragma unroll
+        for (int u = 0; u < kPkU; u++) acc[u] = __builtin_amdgcn_udot4(x[u], x[u], acc[u], false);
+        for (uint32_t q = 0; edge >> q; q++) {
+            if (!(edge >> q & 1)) continue;
+            const uint64_t Sq = q < 2 ? (q ? S[1] : S[0]) : (q == 2 ? S[2] : S[3]);
+#pragma unroll
+            for (int u = 0; u < kPkU; u++) {
+                const uint32_t p = (search_h16(Sq + lane8 + u) * fan) >> 16;
+                acc[u] += p * p;
+            }
+        }
+    }
+}
+
+// Exact test of one candidate of a full-size node: every part has `unit` keys.
+__device__ __forceinline__ bool pk_exact(const uint64_t *kp, uint32_t m, uint32_t fan, uint32_t unit, uint64_t seed) {
+    const uint32_t lane = lane_id();
+    uint32_t cnt[kMaxFanout - 1];
+#pragma unroll
+    for (uint32_t f = 0; f + 1 < kMaxFanout; f++) cnt[f] = 0;
+    for (uint32_t j0 = 0; j0 < m; j0 += 64) {
+        const bool valid = j0 + lane < m;
+        const uint32_t p = valid ? (fold_h16(kp[j0 + lane] + seed) * fan) >> 16 : kMaxFanout;
+#pragma unroll
+        for (uint32_t f = 0; f + 1 < kMaxFanout; f++)
+            if (f + 1 < fan) cnt[f] += (uint32_t)__popcll(__ballot(p == f));
+    }
+    bool ok = true;
+#pragma unroll
+    for (uint32_t f = 0; f + 1 < kMaxFanout; f++)
+        if (f + 1 < fan) ok &= cnt[f] == unit;
+    return ok;
+}
+
+// Class bounds of a node (k_class_order): bound c (1..7) in bits 12 (c - 1).. of the
+// node state's 96 spare bits.
+__device__ __forceinline__ uint32_t pk_bound(uint32_t w0, uint64_t w1, int c) {
+    // bounds 1 and 2 in w0, 3..7 in w1
+    return c <= 2 ? (w0 >> (12 * (c - 1))) & 0xFFF : (uint32_t)(w1 >> (12 * (c - 3))) & 0xFFF;
+}
+
+// One claim of a full-size node: n_groups groups of 512 candidates from x0 on, as
+// staged_claim.
+__device__ __noinline__ uint64_t packed_claim(const uint64_t *kp_any, uint32_t m_any, uint32_t unit_any, uint64_t sconst_any,
+                                              uint64_t x0_any, uint32_t n_groups_any, const NodeState *st_any,
+                                              uint32_t *groups_run) {
+    const uint64_t *kp = (const uint64_t *)uni64((uint64_t)kp_any);
+    const NodeState *st = (const NodeState *)uni64((uint64_t)st_any);
+    const uint32_t m = uni(m_any), unit = uni(unit_any), n_groups = uni(n_groups_any);
+    const uint32_t fan = uni(m / unit), lane8 = lane_id() * 8;
+    const uint64_t x0 = uni64(x0_any), sconst = uni64(sconst_any);
+    const uint32_t w0 = uni(st->pad0);
+    const uint64_t w1 = uni64(st->pad1);
+    uint32_t fan16;
+    __asm__("v_lshlrev_b32 %0, 16, %1" : "=v"(fan16) : "v"(fan));
+    const uint32_t T = unit * ((fan - 1) * fan * (2 * fan - 1) / 6);
+    uint64_t hit = kNone;
+    uint32_t g = 0;
+    for (; g < n_groups && hit == kNone; g++) {
+        const uint64_t xg = x0 + (uint64_t)g * (64 * kPkU);
+        if (g > 0) {
+            unsigned long long r = 0;
+            if (lane_id() == 0) r = ld_relaxed(&st->result);
+            if (xg >= uni64(r)) break;
+        }
+        const uint64_t base = sconst + xg;
+        uint32_t acc[kPkU];
+#pragma unroll
+        for (int u = 0; u < kPkU; u++) acc[u] = 0;
+        const uint32_t c1 = pk_bound(w0, w1, 1), c2 = pk_bound(w0, w1, 2), c3 = pk_bound(w0, w1, 3);
+        const uint32_t c4 = pk_bound(w0, w1, 4), c5 = pk_bound(w0, w1, 5), c6 = pk_bound(w0, w1, 6);
+        const uint32_t c7 = pk_bound(w0, w1, 7);
+        pk_class<0>(kp, 0, c1, base, lane8, fan16, fan, acc);
+        pk_class<1>(kp, c1, c2, base, lane8, fan16, fan, acc);
+        pk_class<2>(kp, c2, c3, base, lane8, fan16, fan, acc);
+        pk_class<3>(kp, c3, c4, base, lane8, fan16, fan, acc);
+        pk_class<4>(kp, c4, c5, base, lane8, fan16, fan, acc);
+        pk_class<5>(kp, c5, c6, base, lane8, fan16, fan, acc);
+        pk_class<6>(kp, c6, c7, base, lane8, fan16, fan, acc);
+        pk_class<7>(kp, c7, m, base, lane8, fan16, fan, acc);
+        // candidates in order: lane by lane, then u
+        unsigned long long any = 0;
+        uint32_t mine = 0;
+#pragma unroll
+        for (int u = 0; u < kPkU; u++) mine |= (acc[u] == T ? 1u : 0u) << u;
+        any = __ballot(mine != 0);
+        while (any && hit == kNone) {
+            const int l = __ffsll((long long)any) - 1;
+            any &= any - 1;
+            uint32_t us = (uint32_t)__builtin_amdgcn_readlane((int)mine, l);
+            while (us && hit == kNone) {
+                const uint64_t x = xg + (uint64_t)l * kPkU + (uint64_t)(__ffs((int)us) - 1);
+                us &= us - 1;
+                if (pk_exact(kp, m, fan, unit, sconst + x)) hit = x;
+            }
+        }
+    }
+    *groups_run = g;
+    return hit;
+}
+
 // Rotation leaves of at most this many keys test candidates through the table of
 // least rotations (2^L two-byte entries of LDS).
 constexpr uint32_t kNecklaceMax = 12;
@@ -1064,8 +1285,8 @@ __device__ __forceinline__ bool has_work(const NodeState *st, uint64_t units_per
 // (aggregation levels and rotation leaves below kStagedMinLeaf, 16-bit remap): the
 // byte table for nodes of bt_m keys, workgroups of kBtThreads threads, two per CU
 // (registers held to the kBtThreads / 128 waves per SIMD that two such workgroups need).
-template <int KIND, int U, bool WIDE, bool LUT, bool SK, bool R64, bool ST = false, bool BT = false>
-__global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) / 128 : (KIND == kLeafRot ? 5 : 1)) void k_search(const uint64_t *__restrict__ keys,
+template <int KIND, int U, bool WIDE, bool LUT, bool SK, bool R64, bool ST = false, bool BT = false, bool PK = false>
+__global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) / 128 : (PK ? 8 : KIND == kLeafRot ? 5 : 1)) void k_search(const uint64_t *__restrict__ keys,
                                                                                   SearchArgs a) {
     static_assert(!BT || ((((KIND == kUpper || KIND == kLower) && LUT) || KIND == kLeafRot) && !R64 && !ST),
                   "the byte table serves aggregation levels and rotation leaves over the 16-bit remap");
@@ -1323,7 +1544,13 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
                 work += (uint64_t)groups_run * U * 64 * k + (uint64_t)tests_run * 64 * (m - k);
             }
         }
-        const bool single = !ST || (KIND == kLeafBrute && m < kStagedMinLeaf);
+        const bool packed = PK && m == a.bt_m;
+        if (packed) {
+            uint32_t groups_run;
+            hit = packed_claim(kp, m, a.split_unit, sconst, unit0, a.groups * span, &a.state[node], &groups_run);
+            work += (uint64_t)groups_run * U * 64 * m;
+        }
+        const bool single = !packed && (!ST || (KIND == kLeafBrute && m < kStagedMinLeaf));
         for (uint32_t g = 0; single && g < a.groups * span; g++) {
             const uint64_t u0 = unit0 + (uint64_t)g * U * 64;
             if (g > 0) {
@@ -1336,7 +1563,13 @@ __global__ __launch_bounds__(BT ? bt_threads(KIND) : 256, BT ? bt_threads(KIND) 
             if (KIND == kHigher) hit = group_higher<U, SK, R64>(kp, m, sconst, aux0, aux1, u0);
             else if ((KIND == kUpper || KIND == kLower) && BT && m == a.bt_m)
                 hit = group_aggr_bt<U, SK, WIDE>(kp, m, sconst, bt_table<BT>(), T, cmask, u0);
-            else if (KIND == kUpper || KIND == kLower)
+            else if (PK) {
+                // other sizes of the level: the increment table, four candidates per lane
+                hit = group_aggr<4, WIDE, LUT, SK, R64>(kp, m, sconst, a.field_bits, a.magic, T, cmask, lut_hi, two, u0);
+                if (hit == kNone)
+                    hit = group_aggr<4, WIDE, LUT, SK, R64>(kp, m, sconst, a.field_bits, a.magic, T, cmask, lut_hi, two,
+                                                            u0 + 256);
+            } else if (KIND == kUpper || KIND == kLower)
                 hit = group_aggr<U, WIDE, LUT, SK, R64>(kp, m, sconst, a.field_bits, a.magic, T, cmask, lut_hi, two,
                                                         u0);
             else if (KIND == kLeafRot && !ST)
@@ -1368,6 +1601,76 @@ __global__ __launch_bounds__(256) void k_state_init(NodeState *st, uint32_t n) {
         st[i].result = kNone;
         st[i].next_chunk = 1;  // chunk 0 is taken by the wave that starts the node
         st[i].waves = 0;
+    }
+}
+
+// Search state of a level whose full-size nodes (full_m keys) run packed: initial
+// values, and the node's keys ordered in place by (key + start seed) mod 8, with the
+// class bounds in the state's spare bits.  One wavefront per node, keys staged in
+// LDS; 16 B of traffic per key, once per level.
+__global__ __launch_bounds__(64) void k_class_order(uint64_t *__restrict__ keys, const NodeDesc *__restrict__ nodes,
+                                                    NodeState *__restrict__ st, uint32_t n_nodes, uint32_t full_m,
+                                                    uint32_t seed_index, const uint64_t *__restrict__ count_dev = nullptr,
+                                                    const uint64_t *__restrict__ lbase_dev = nullptr, uint32_t list = 0) {
+    extern __shared__ uint64_t s_keys[];
+    if (count_dev) {
+        n_nodes = (uint32_t)count_dev[list];
+        nodes += lbase_dev[list];
+    }
+    const uint32_t lane = threadIdx.x;
+    const uint32_t c3 = (uint32_t)c_start_seed[seed_index];
+    const unsigned long long lt = (1ull << lane) - 1;
+    for (uint32_t i = blockIdx.x; i < n_nodes; i += gridDim.x) {
+        const NodeDesc d = nodes[i];
+        uint64_t w1 = 0;
+        uint32_t w0 = 0;
+        if (d.m == full_m) {
+            uint64_t *kp = keys + d.key_off;
+            uint32_t fill[8];
+#pragma unroll
+            for (int c = 0; c < 8; c++) fill[c] = 0;
+            for (uint32_t j0 = 0; j0 < full_m; j0 += 64) {
+                const bool valid = j0 + lane < full_m;
+                const uint64_t k = valid ? kp[j0 + lane] : 0;
+                if (valid) s_keys[j0 + lane] = k;
+                const uint32_t cls = ((uint32_t)k + c3) & 7;
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++) fill[c] += (uint32_t)__popcll(__ballot(valid && cls == c));
+            }
+            uint32_t run = 0;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const uint32_t f = fill[c];
+                fill[c] = run;
+                if (c == 1 || c == 2) w0 |= run << (12 * (c - 1));
+                if (c >= 3) w1 |= (uint64_t)run << (12 * (c - 3));
+                run += f;
+            }
+            __syncthreads();
+            for (uint32_t j0 = 0; j0 < full_m; j0 += 64) {
+                const bool valid = j0 + lane < full_m;
+                const uint64_t k = valid ? s_keys[j0 + lane] : 0;
+                const uint32_t cls = ((uint32_t)k + c3) & 7;
+                uint32_t at = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++) {
+                    const unsigned long long b = __ballot(valid && cls == c);
+                    if (cls == c) at = fill[c] + (uint32_t)__popcll(b & lt);
+                    fill[c] += (uint32_t)__popcll(b);
+                }
+                if (valid) kp[at] = k;
+            }
+            __syncthreads();  // s_keys is reused by the next node
+        }
+        if (lane == 0) {
+            NodeState n;
+            n.result = kNone;
+            n.next_chunk = 1;  // chunk 0 is taken by the wave that starts the node
+            n.waves = 0;
+            n.pad0 = w0;
+            n.pad1 = w1;
+            st[i] = n;
+        }
     }
 }
 

@@ -212,6 +212,7 @@ struct rs_plan {
     std::vector<int> lists;     // tree levels some bucket size can have
     std::vector<char> likely;   // ... and whether a bucket of the likely sizes has it
     std::vector<uint32_t> level_blocks;  // ... and its search grid (expected work)
+    std::vector<double> level_nodes;     // ... and its expected nodes
     std::vector<char> mostly_full;       // ... and whether most of its nodes are of full size
     uint32_t likely_max_bucket = 0;  // bucket sizes above this are vanishingly rare
     // device buffers
@@ -335,12 +336,19 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
             if (!lut) lds = 0;
         }
         const SearchShape sh =
-            search_shape(tn, kind, wide, lut, r64, p->mostly_full[li] != 0, blocks, p->blocks, (uint32_t)p->num_cus, P.leaf);
-        a.bt_m = sh.bt ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
+            search_shape(tn, kind, wide, lut, r64, p->mostly_full[li] != 0, blocks, p->blocks, (uint32_t)p->num_cus, P.leaf,
+                         lds ? golomb_param(golomb_memo(P.leaf), a.lut_entries) : 0, p->level_nodes[li]);
+        a.bt_m = sh.bt || sh.pk ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
         a.n_waves = sh.waves;
         k_level_init<<<likely ? fill_grid : 4, 256, 0, s>>>(p->state, p->running, p->ctl, sh.waves, p->list_count,
                                                             (uint32_t)l);
-        launch_search(s, tn, kind, p->sorted, a, wide, lut, sh.grid, lds, r64);
+        if (sh.pk) {
+            a.groups = 1;
+            k_class_order<<<likely ? (uint32_t)p->num_cus * 8 : 8, 64, (size_t)a.bt_m * 8, s>>>(
+                p->sorted, p->pool, p->state, 0, a.bt_m, kind == kUpper ? kSeedUpper : kSeedLower, p->list_count,
+                p->list_base, (uint32_t)l);
+        }
+        launch_search(s, tn, kind, p->sorted, a, wide, lut, sh.grid, lds, r64, sh.pk);
         if (kind == kHigher || kind == kUpper || kind == kLower) {
             const uint32_t max_m = kind == kHigher ? kMaxBucket : (kind == kUpper ? P.upper : P.lower);
             k_split<<<likely ? (uint32_t)p->num_cus * 8 : 8, 64, (size_t)max_m * 8, s>>>(
@@ -487,6 +495,7 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
                 p->lists.push_back(l);
                 p->likely.push_back(lik ? 1 : 0);
                 p->level_blocks.push_back(rsa::level_blocks(e * (double)NB, cnt * (double)NB, p->blocks));
+                p->level_nodes.push_back(cnt * (double)NB);
                 p->mostly_full.push_back(2 * nfull >= cnt ? 1 : 0);
             }
         }

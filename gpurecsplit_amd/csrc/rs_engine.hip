@@ -29,6 +29,7 @@
 
 #include "rs_internal.h"
 #include "rs_kernels.hip"
+#include "rs_tree.hip"
 
 namespace rsa {
 
@@ -195,6 +196,7 @@ struct Census {
     uint64_t count[kNumLists] = {};
     double evals[kNumLists] = {};
     uint64_t full[kNumLists] = {};  // aggregation nodes of the level's full size
+    double most[kNumLists] = {};    // expected key evaluations of the list's heaviest node
     uint32_t max_depth = 0;
 };
 
@@ -205,6 +207,7 @@ struct SubCensus {
     uint64_t n[4] = {};
     double e[4] = {};
     uint64_t f[4] = {};
+    double x[4] = {};
 };
 
 // Expected key evaluations of the search of one node of s keys.  The Golomb-Rice
@@ -226,6 +229,7 @@ static void census_node(const SplitParams &P, const Memo &memo, bool rotate, uin
             SubCensus acc;
             acc.n[kind - 1] += 1;
             acc.e[kind - 1] += node_evals(memo, s, kind, P.leaf);
+            acc.x[kind - 1] = acc.e[kind - 1];
             acc.f[kind - 1] += (kind == kUpper && s == P.upper) || (kind == kLower && s == P.lower);
             if (s > P.leaf) {
                 const uint32_t unit = kind == kUpper ? P.lower : P.leaf;
@@ -239,6 +243,7 @@ static void census_node(const SplitParams &P, const Memo &memo, bool rotate, uin
                             acc.n[k] += part.count[kMaxDepth + k];
                             acc.e[k] += part.evals[kMaxDepth + k];
                             acc.f[k] += part.full[kMaxDepth + k];
+                            acc.x[k] = std::max(acc.x[k], part.most[kMaxDepth + k]);
                         }
                     }
                 }
@@ -250,12 +255,14 @@ static void census_node(const SplitParams &P, const Memo &memo, bool rotate, uin
             c.count[kMaxDepth + k] += sub.n[k] * mult;
             c.evals[kMaxDepth + k] += sub.e[k] * (double)mult;
             c.full[kMaxDepth + k] += sub.f[k] * mult;
+            c.most[kMaxDepth + k] = std::max(c.most[kMaxDepth + k], sub.x[k]);
         }
         return;
     }
     if (depth >= kMaxDepth) throw BuildError(RS_ERR_ARG, "split tree deeper than the start-seed table");
     c.count[depth] += mult;
     c.evals[depth] += node_evals(memo, s, kHigher, P.leaf) * (double)mult;
+    c.most[depth] = std::max(c.most[depth], node_evals(memo, s, kHigher, P.leaf));
     c.max_depth = std::max(c.max_depth, depth);
     const uint32_t split = higher_split(P, s);
     census_node(P, memo, rotate, split, depth + 1, mult, c, small);
@@ -307,6 +314,7 @@ struct Tune {
     // fanout-2 nodes need ~40 candidates, so extra waves mostly overshoot
     int help_cap[kNumKinds] = {2, 0, 0, 0, 0};
     int blocks_per_cu = 8;
+    int tree = 1;    // whole trees of small buckets in one kernel
     int pk = 1;      // packed parts for the full-size nodes of heavy aggregation levels
     int bt = 1;      // byte table for the full-size nodes of aggregation levels
     int u_bt = 4;    // candidates in flight per lane in those launches
@@ -333,6 +341,7 @@ static Tune parse_tune(const char *env, Tune t = Tune()) {
             else if (k.size() == 2 && k[0] == 'u' && k[1] >= '0' && k[1] < '0' + (int)kNumKinds && uv)
                 t.u[k[1] - '0'] = v;
             else if (k == "lut") t.lut = v != 0;
+            else if (k == "tree") t.tree = v != 0;
             else if (k == "pk") t.pk = v != 0;
             else if (k == "bt") t.bt = v != 0;
             else if (k == "ubt" && uv) t.u_bt = v;
@@ -363,6 +372,7 @@ static std::string format_tune(const Tune &t) {
     for (int k = 0; k < kNumKinds; k++) add("sk" + std::to_string(k), t.sk[k]);
     for (int k = 0; k < kNumKinds; k++) add("h" + std::to_string(k), t.help_cap[k]);
     add("lut", t.lut);
+    add("tree", t.tree);
     add("pk", t.pk);
     add("bt", t.bt);
     add("ubt", t.u_bt);
@@ -606,6 +616,66 @@ static void launch_search(hipStream_t s, const Tune &tn, uint32_t kind, const ui
     HIP_CHECK(hipGetLastError());
 }
 
+// Expected work of a build, summed over its lists.
+struct TreeWork {
+    double evals = 0, nodes = 0;
+    double tail = 0;  // key evaluations of the longest search: a list's heaviest node times ln(1 + its nodes)
+    void add(double list_evals, double list_nodes, double most) {
+        evals += list_evals;
+        nodes += list_nodes;
+        tail = std::max(tail, most * std::log1p(list_nodes));
+    }
+};
+
+// Whether a build's buckets run as whole trees (k_tree).  A bucket's keys must fit a
+// share of LDS and the packed counters 32 bits.  One wave searches a node, so the
+// tree kernel cannot end before the longest search, 0.32 ns per expected evaluation
+// of `tail` (a wave hashes 64 keys in about 50 cycles), nor before a bucket's own
+// evaluations (shared by four waves where buckets are few).  The level kernels'
+// launches, syncs and per-node atomics cost about 0.6 ms and 18 ns per node beside the
+// evaluations that both do.  Both sides measured at 1K to 3M keys, l = 4..16: 1M keys
+// at l = 8, b = 100 4.4 ms by levels, 1.1 as trees; l = 12, b = 100 4.4 and 2.4;
+// 1M keys at l = 14, b = 20 8.6 and 5.9, but 100K of them 2.0 and 2.4.
+constexpr uint32_t kTreeMaxBucket = 512;
+static bool tree_fits(const Tune &tn, const AggrLayout &up, const AggrLayout &lo, uint32_t max_bucket,
+                      const TreeWork &w, double buckets, uint32_t num_cus) {
+    if (!tn.tree || up.wide || lo.wide || max_bucket > kTreeMaxBucket) return false;
+    const double chain = w.evals / buckets / (buckets <= 8.0 * num_cus ? 4 : 1);
+    return 0.32e-9 * std::max(w.tail, chain) <= 0.6e-3 + 18e-9 * w.nodes;
+}
+
+// Candidates per lane of the lower level and the leaves: one where a node's expected
+// candidates are few (its overshoot is half a group of 64 * U).
+template <int U>
+static void launch_tree_u(hipStream_t s, const TreeArgs &a, uint32_t blocks, uint32_t threads, size_t lds, bool r64,
+                          bool team) {
+    if (team) {
+        if (r64) k_tree<U, true, true><<<blocks, threads, lds, s>>>(a);
+        else k_tree<U, false, true><<<blocks, threads, lds, s>>>(a);
+    } else {
+        if (r64) k_tree<U, true, false><<<blocks, threads, lds, s>>>(a);
+        else k_tree<U, false, false><<<blocks, threads, lds, s>>>(a);
+    }
+}
+static uint32_t launch_tree(hipStream_t s, TreeArgs a, bool r64, uint32_t num_cus) {
+    // a workgroup per bucket while one wave per bucket would not fill the SIMDs
+    // a launch for oversized buckets only (cap above kTreeMaxBucket) always does
+    const bool team = a.nb <= 8 * num_cus || a.cap > kTreeMaxBucket;
+    const uint32_t wpg = team && a.nb <= 2 * num_cus ? 8 : 4;
+    const TreeLds l = tree_lds(a.P, a.rotate != 0, a.cap, wpg, team);
+    a.scratch = l.scratch;
+    a.queue = l.queue;
+    const uint64_t resident = std::max<uint64_t>(1, std::min<uint64_t>(32 / wpg, (160u << 10) / (l.bytes + 4096)));
+    const uint64_t groups = team ? a.nb : (a.nb + wpg - 1) / wpg;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(groups, num_cus * resident);
+    a.batch = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, a.nb / ((uint64_t)blocks * wpg * 16)));
+    if (a.P.leaf <= 8) launch_tree_u<1>(s, a, blocks, wpg * 64, l.bytes, r64, team);
+    else if (a.P.leaf <= 10) launch_tree_u<2>(s, a, blocks, wpg * 64, l.bytes, r64, team);
+    else launch_tree_u<4>(s, a, blocks, wpg * 64, l.bytes, r64, team);
+    HIP_CHECK(hipGetLastError());
+    return blocks * wpg;
+}
+
 __global__ void k_gather_u64(const uint64_t *__restrict__ src, const uint64_t *__restrict__ idx, uint64_t n,
                              uint64_t *__restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -772,38 +842,53 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     HIP_CHECK(hipMemsetAsync(cursor, 0, NB * 4, s));
     k_scatter<<<tiles.size(), 256, (size_t)priv_max * 4, s>>>(d_tiles, acc, cursor, sorted, priv_max);
     HIP_CHECK(hipGetLastError());
-    uint32_t sort_p = 1;
-    while (sort_p < st.max_bucket_size) sort_p <<= 1;
-    k_sort_buckets<<<NB, st.max_bucket_size > 512 ? 256 : 64, (size_t)sort_p * 8, s>>>(sorted, acc, err,
-                                                                                       rotate ? leaf : 0);
-    HIP_CHECK(hipGetLastError());
+    const Tune tn = tune_for(c, leaf);
+    const AggrLayout up_l = aggr_layout(P.lower, P.upper / P.lower);
+    const AggrLayout lo_l = aggr_layout(P.leaf, P.lower / P.leaf);
+    TreeWork tw;
+    for (int l = 0; l < kNumLists; l++) tw.add(cen.evals[l], (double)cen.count[l], cen.most[l]);
+    const bool tree = !(c->wave_times && !t_arena) &&
+                      tree_fits(tn, up_l, lo_l, st.max_bucket_size, tw, (double)NB, (uint32_t)c->num_cus);
+    if (!tree) {
+        uint32_t sort_p = 1;
+        while (sort_p < st.max_bucket_size) sort_p <<= 1;
+        k_sort_buckets<<<NB, st.max_bucket_size > 512 ? 256 : 64, (size_t)sort_p * 8, s>>>(sorted, acc, err,
+                                                                                           rotate ? leaf : 0);
+        HIP_CHECK(hipGetLastError());
+    }
 
     // ---- 3. node lists
     const uint64_t pool_n = std::max<uint64_t>(total_nodes, 1);
-    NodeDesc *pool = c->pool.get<NodeDesc>(pool_n);
-    uint64_t *d_lbase = c->list_base.get<uint64_t>(kNumLists);
-    uint32_t *d_lfill = c->list_fill.get<uint32_t>(kNumLists);
     uint16_t *node_m = c->node_m.get<uint16_t>(pool_n);
     uint64_t *seeds = c->seeds.get<uint64_t>(pool_n);
-    HIP_CHECK(hipMemcpyAsync(d_lbase, lbase.data(), kNumLists * 8, hipMemcpyHostToDevice, s));
-    HIP_CHECK(hipMemsetAsync(d_lfill, 0, kNumLists * 4, s));
-    ExpandArgs ea{P, rotate ? 1 : 0, pool, d_lbase, d_lfill, node_m};
-    k_expand<<<(NB + 63) / 64, 64, 0, s>>>(acc, node_base, NB, ea);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(h, err, 4, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync((uint64_t *)h + 1, node_base + NB, 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (h[0] & 1) throw BuildError(RS_ERR_DUPLICATE_KEYS, "two keys of one bucket share the same `second` half");
-    if (((uint64_t *)h)[1] != total_nodes)
-        throw BuildError(RS_ERR_INTERNAL, "seed slots " + std::to_string(((uint64_t *)h)[1]) + " != tree nodes " +
-                                              std::to_string(total_nodes));
+    NodeDesc *pool = nullptr;
+    auto check_partition = [&](uint32_t err_word, uint64_t slots) {
+        if (err_word & kErrDuplicateKeys)
+            throw BuildError(RS_ERR_DUPLICATE_KEYS, "two keys of one bucket share the same `second` half");
+        if (slots != total_nodes)
+            throw BuildError(RS_ERR_INTERNAL, "seed slots " + std::to_string(slots) + " != tree nodes " +
+                                                  std::to_string(total_nodes));
+    };
+    if (!tree) {
+        pool = c->pool.get<NodeDesc>(pool_n);
+        uint64_t *d_lbase = c->list_base.get<uint64_t>(kNumLists);
+        uint32_t *d_lfill = c->list_fill.get<uint32_t>(kNumLists);
+        HIP_CHECK(hipMemcpyAsync(d_lbase, lbase.data(), kNumLists * 8, hipMemcpyHostToDevice, s));
+        HIP_CHECK(hipMemsetAsync(d_lfill, 0, kNumLists * 4, s));
+        ExpandArgs ea{P, rotate ? 1 : 0, pool, d_lbase, d_lfill, node_m};
+        k_expand<<<(NB + 63) / 64, 64, 0, s>>>(acc, node_base, NB, ea);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipMemcpyAsync(h, err, 4, hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipMemcpyAsync((uint64_t *)h + 1, node_base + NB, 8, hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipStreamSynchronize(s));
+        check_partition(h[0], ((uint64_t *)h)[1]);
+    }
     const int e_part1 = ev_record(c);
 
     // ---- 4. search phases
     uint64_t max_list = 1;
-    for (int l = 0; l < kNumLists; l++) max_list = std::max(max_list, cen.count[l]);
+    for (int l = 0; l < kNumLists && !tree; l++) max_list = std::max(max_list, cen.count[l]);
     NodeState *state = c->state.get<NodeState>(max_list);
-    const Tune tn = tune_for(c, leaf);
     const uint32_t blocks = (uint32_t)c->num_cus * (uint32_t)tn.blocks_per_cu;
     const uint32_t n_waves = blocks * 4;
     st.search_waves = n_waves;
@@ -816,14 +901,45 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         wave_clock = c->wave_clock.get<unsigned long long>((size_t)kNumLists * 2 * n_waves);
         HIP_CHECK(hipMemsetAsync(wave_clock, 0, (size_t)kNumLists * 2 * n_waves * 8, s));
     }
-    const AggrLayout up_l = aggr_layout(P.lower, P.upper / P.lower);
-    const AggrLayout lo_l = aggr_layout(P.leaf, P.lower / P.leaf);
+    uint64_t *bits = c->bits.get<uint64_t>(NB);
+    unsigned long long *evals = c->evals.get<unsigned long long>(2 * kNumKinds);  // evaluations, then seeds
+    HIP_CHECK(hipMemsetAsync(evals, 0, 2 * kNumKinds * 8, s));
     struct PhaseEvents {
         uint32_t kind;
         int search0, search1, split1;
     };
     std::vector<PhaseEvents> phase_ev;
-    for (int l = 0; l < kNumLists; l++) {
+    if (tree) {
+        // the whole trees, one wave per bucket; work counters by kind in work[0, kNumKinds)
+        HIP_CHECK(hipMemsetAsync(ctl, 0, 64, s));
+        TreeArgs a{};
+        a.acc = acc;
+        a.node_base = node_base;
+        a.sorted = sorted;
+        a.seeds = seeds;
+        a.node_m = node_m;
+        a.bits = bits;
+        a.evals = evals;
+        a.work = work;
+        a.memo = memo;
+        a.err = err;
+        a.ctl = ctl;
+        a.nb = NB;
+        a.P = P;
+        a.rotate = rotate ? 1 : 0;
+        a.max_m = st.max_bucket_size;
+        a.cap = std::max<uint32_t>(64, (st.max_bucket_size + 7) & ~7u);
+        a.up_fb = up_l.fb;
+        a.up_magic = up_l.magic;
+        a.lo_fb = lo_l.fb;
+        a.lo_magic = lo_l.magic;
+        a.clock0 = clock0;
+        a.limit_ticks = limit_ticks;
+        const uint32_t waves = launch_tree(s, a, r64, (uint32_t)c->num_cus);
+        for (int k = 0; k < kNumKinds; k++)
+            if (st.nodes[k]) st.kind_waves[k] = waves;
+    }
+    for (int l = 0; l < kNumLists && !tree; l++) {
         const uint32_t cnt = (uint32_t)cen.count[l];
         if (!cnt) continue;
         const uint32_t kind = l < (int)kMaxDepth ? kHigher : (uint32_t)(l - kMaxDepth + 1);
@@ -895,13 +1011,13 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     const int e_search_end = ev_record(c);
 
     // ---- 5. descriptor lengths (global scan; each set reads its segment)
-    uint64_t *bits = c->bits.get<uint64_t>(NB);
     uint64_t *pos = c->pos.get<uint64_t>(NB + 1);
-    unsigned long long *evals = c->evals.get<unsigned long long>(2 * kNumKinds);  // evaluations, then seeds
-    HIP_CHECK(hipMemsetAsync(evals, 0, 2 * kNumKinds * 8, s));
     EncodeArgs ca{acc, node_base, seeds, node_m, memo, memo + kMaxBucket, NB, P, rotate ? 1 : 0};
-    k_bucket_bits<<<(uint32_t)std::min<uint64_t>((NB + 3) / 4, (uint64_t)c->num_cus * 8), 256, 0, s>>>(ca, bits, evals);
-    HIP_CHECK(hipGetLastError());
+    if (!tree) {
+        k_bucket_bits<<<(uint32_t)std::min<uint64_t>((NB + 3) / 4, (uint64_t)c->num_cus * 8), 256, 0, s>>>(ca, bits,
+                                                                                                          evals);
+        HIP_CHECK(hipGetLastError());
+    }
     scan_u64(c, bits, false, NB, pos);
     uint64_t *d_bidx = c->set_idx.get<uint64_t>(S + 1);
     uint64_t *d_gath = c->set_gather.get<uint64_t>(S + 1);
@@ -916,16 +1032,20 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     HIP_CHECK(hipMemcpyAsync(h64 + 64, evals, 2 * kNumKinds * 8, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipMemcpyAsync(h64 + 16, work, kNumLists * 8, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipMemcpyAsync(h + 16, err, 4, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(h64 + 80, node_base + NB, 8, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
+    if (h[16] & kErrTimeout)
+        throw BuildError(RS_ERR_TIMEOUT, "the build passed the context's time limit during the seed search");
+    if (tree) check_partition(h[16], h64[80]);
     for (int k = 0; k < kNumKinds; k++) {
         st.evals[k] = h64[64 + k];
         st.seeds[k] = h64[64 + kNumKinds + k];
     }
     static_assert(16 + kNumLists <= 64, "work counters overlap the evaluation counts");
-    for (int l = 0; l < kNumLists; l++)
+    for (int l = 0; l < kNumLists && !tree; l++)
         st.executed_evals[l < (int)kMaxDepth ? kHigher : l - kMaxDepth + 1] += h64[16 + l];
+    for (int k = 0; k < kNumKinds && tree; k++) st.executed_evals[k] = h64[16 + k];
     if (wave_clock) wave_time_stats(c, wave_clock, n_waves, cen.count, st);
-    if (h[16] & 8) throw BuildError(RS_ERR_TIMEOUT, "the build passed the context's time limit during the seed search");
     if (h[16] & 2) throw BuildError(RS_ERR_SEED_OVERFLOW, "a node search passed the 2^44 seed limit");
 
     // ---- 6. Golomb-Rice: per-set vectors packed one after another
@@ -1085,6 +1205,13 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         st.search_ms[pe.kind] += ev_ms(c, pe.search0, pe.search1);
         st.split_ms += ev_ms(c, pe.search1, pe.split1);
     }
+    if (tree) {
+        // one launch searches every kind: its time by the kinds' executed evaluations
+        double all = 0;
+        for (int k = 0; k < kNumKinds; k++) all += (double)st.executed_evals[k];
+        for (int k = 0; k < kNumKinds && all > 0; k++)
+            st.search_ms[k] = ev_ms(c, e_part1, e_search_end) * (double)st.executed_evals[k] / all;
+    }
     st.encode_ms = ev_ms(c, e_search_end, e_enc_end);
     st.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
 
@@ -1179,7 +1306,9 @@ __global__ __launch_bounds__(256) void k_splitmix_keys(uint64_t seed, uint64_t n
 // the sample is sized so that a build takes about 40 ms.  The result becomes
 // the context's tuning for the leaf size.  Returns a JSON report.
 static std::string autotune(rs_ctx *c, uint32_t leaf, uint64_t bucket, int flags, uint64_t sample_keys) {
-    const Tune base = tune_for(c, leaf);
+    Tune base = tune_for(c, leaf);
+    const int tree = base.tree;
+    base.tree = 0;  // the settings under trial are those of the level kernels
     c->tuned[leaf] = true;  // builds below run with explicit tunings (no recursion)
     const uint64_t n_max = uint64_t(1) << 22;
     uint64_t *keys = c->tune_keys.get<uint64_t>(2 * n_max);
@@ -1265,6 +1394,7 @@ static std::string autotune(rs_ctx *c, uint32_t leaf, uint64_t bucket, int flags
             best.blocks_per_cu = b;
         }
     }
+    best.tree = tree;
     c->tune_leaf[leaf] = best;
     rep += "],\"search_ms_after\":" + std::to_string(best_total) + ",\"tune\":\"" + format_tune(best) + "\"}";
     return rep;

@@ -489,6 +489,41 @@ __device__ __forceinline__ void stream_keys_scalar(const uint64_t *__restrict__ 
     }
 }
 
+// Streams keys of LDS (kp[begin, end), wave-uniform bounds): each lane holds one key of
+// 64, and a lane read per key puts it into scalar registers.
+template <typename F>
+__device__ __forceinline__ void stream_keys_lds(const uint64_t *kp_any, uint32_t begin_any, uint32_t end_any, F &&f) {
+    typedef const __attribute__((address_space(3))) uint64_t *lds_keys;
+    const lds_keys kp = (lds_keys)(uintptr_t)(uint32_t)(uintptr_t)kp_any;
+    const uint32_t end = uni(end_any), lane = lane_id();
+    auto key = [](uint64_t k, uint32_t j) -> uint64_t {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, (int)j);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(k >> 32), (int)j);
+        return ((uint64_t)hi << 32) | lo;
+    };
+    for (uint32_t j0 = uni(begin_any); j0 < end; j0 += 64) {
+        const uint32_t cnt = end - j0 < 64 ? end - j0 : 64;
+        const uint64_t k = kp[j0 + (lane < cnt ? lane : cnt - 1)];
+        uint32_t j = 0;
+        for (; j + 4 <= cnt; j += 4) {
+            f(key(k, j));
+            f(key(k, j + 1));
+            f(key(k, j + 2));
+            f(key(k, j + 3));
+        }
+        for (; j < cnt; j++) f(key(k, j));
+    }
+}
+
+// Where a search reads its node's keys: vector loads, scalar loads, or LDS.
+constexpr int kKeysVector = 0, kKeysScalar = 1, kKeysLds = 2;
+
+template <int SK, typename F>
+__device__ __forceinline__ void stream_keys_uniform(const uint64_t *__restrict__ kp, uint32_t begin, uint32_t end, F &&f) {
+    if constexpr (SK == kKeysLds) stream_keys_lds(kp, begin, end, f);
+    else stream_keys_scalar(kp, begin, end, f);
+}
+
 // Candidate seeds of one group: lane-u candidate = base + off[u] (mod 2^64), base
 // wave-uniform, off[u] < 2^32 per lane, max_off >= every off[u].
 template <int U>
@@ -515,13 +550,13 @@ struct Seeds {
 // Past a 2^16 boundary but not a 2^32 one, t is (lo + off) ^ hi; otherwise (within
 // max_off of a 2^32 boundary) the full 64-bit add.  Without SK: vector key
 // loads and per-lane 64-bit seeds.
-template <int U, bool SK, typename G>
+template <int U, int SK, typename G>
 __device__ __forceinline__ void each_hash(const uint64_t *__restrict__ kp, uint32_t begin, uint32_t end,
                                           const Seeds<U> &sd, G &&g) {
-    if (SK) {
+    if constexpr (SK != kKeysVector) {
         const uint64_t base = uni64(sd.base);
         const uint32_t max_off = uni(sd.max_off);
-        stream_keys_scalar(kp, begin, end, [&](uint64_t k) {
+        stream_keys_uniform<SK>(kp, begin, end, [&](uint64_t k) {
             const uint64_t S = k + base;
             const uint32_t lo = (uint32_t)S, hi = (uint32_t)(S >> 32);
             if ((lo & 0xFFFFu) <= 0xFFFFu - max_off) {
@@ -549,11 +584,11 @@ __device__ __forceinline__ void each_hash(const uint64_t *__restrict__ kp, uint3
 
 // 64-bit-remap form of each_hash: calls g(u, r) with r = remap64(key + base +
 // off[u], m) (rs_common.h), keys in scalar registers.
-template <int U, typename G>
+template <int U, int SK, typename G>
 __device__ __forceinline__ void each_r64(const uint64_t *__restrict__ kp, uint32_t begin, uint32_t end,
                                          const Seeds<U> &sd, uint32_t m, G &&g) {
     const uint64_t base = uni64(sd.base);
-    stream_keys_scalar(kp, begin, end, [&](uint64_t k) {
+    stream_keys_uniform<SK>(kp, begin, end, [&](uint64_t k) {
         const uint64_t S = k + base;
 #pragma unroll
         for (int u = 0; u < U; u++) g(u, remap64(S + sd.off[u], m));
@@ -562,14 +597,14 @@ __device__ __forceinline__ void each_r64(const uint64_t *__restrict__ kp, uint32
 
 // Fanout-2 node: lowest x with #{remap(k+S[depth]+x, m) < split} == split
 // (SIMDRecSplit.hpp:250-317).  remap < split <=> h16 < ceil(split*2^16/m).
-template <int U, bool SK, bool R64>
+template <int U, int SK, bool R64>
 __device__ __forceinline__ uint64_t group_higher(const uint64_t *__restrict__ kp, uint32_t m, uint64_t sconst,
                                                  uint32_t split, uint32_t H, uint64_t u0) {
     uint32_t cnt[U];
 #pragma unroll
     for (int u = 0; u < U; u++) cnt[u] = 0;
     if constexpr (R64)
-        each_r64<U>(kp, 0, m, Seeds<U>(u0 + sconst, 1), m, [&](int u, uint32_t r) { cnt[u] += r < split; });
+        each_r64<U, SK>(kp, 0, m, Seeds<U>(u0 + sconst, 1), m, [&](int u, uint32_t r) { cnt[u] += r < split; });
     else
         each_hash<U, SK>(kp, 0, m, Seeds<U>(u0 + sconst, 1), [&](int u, uint32_t h) { cnt[u] += h < H; });
 #pragma unroll
@@ -586,7 +621,7 @@ __device__ __forceinline__ uint64_t group_higher(const uint64_t *__restrict__ kp
 // forces another count negative, so equality of the counted fields is
 // equality of all counts.  With LUT, the increment 1 << (fb * part) of every
 // remapped value r < m is read from the workgroup's LDS table instead of computed.
-template <int U, bool WIDE, bool LUT, bool SK, bool R64>
+template <int U, bool WIDE, bool LUT, int SK, bool R64>
 __device__ __forceinline__ uint64_t group_aggr(const uint64_t *__restrict__ kp, uint32_t m, uint64_t sconst,
                                                uint32_t fb, uint32_t magic, uint64_t T, uint64_t cmask,
                                                uint32_t lut_hi, uint32_t two, uint64_t u0) {
@@ -598,7 +633,7 @@ __device__ __forceinline__ uint64_t group_aggr(const uint64_t *__restrict__ kp, 
     if constexpr (R64) {
         // LDS table at entry lut_hi >> 16, indexed by the remapped value
         const uint32_t lut_b = (lut_hi >> 16) * (uint32_t)sizeof(LutT);
-        each_r64<U>(kp, 0, m, Seeds<U>(u0 + sconst, 1), m, [&](int u, uint32_t r) {
+        each_r64<U, SK>(kp, 0, m, Seeds<U>(u0 + sconst, 1), m, [&](int u, uint32_t r) {
             if (LUT) {
                 cnt[u] += *(const __attribute__((address_space(3))) LutT *)(uintptr_t)(lut_b + (uint32_t)sizeof(LutT) * r);
             } else {
@@ -654,7 +689,7 @@ __device__ __forceinline__ const uint8_t *bt_table() {
 
 // Aggregation node of the byte table's size: the same predicate as group_aggr,
 // the increment of every key 1 << bt[h16] (h16 < 2^16; 64-bit counters for WIDE).
-template <int U, bool SK, bool WIDE>
+template <int U, int SK, bool WIDE>
 __device__ __forceinline__ uint64_t group_aggr_bt(const uint64_t *__restrict__ kp, uint32_t m, uint64_t sconst,
                                                   const uint8_t *bt, uint64_t T, uint64_t cmask, uint64_t u0) {
     using C = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
@@ -907,7 +942,7 @@ constexpr uint32_t kNecklaceMax = 12;
 // makes both halves collision-free: a collision changes a popcount), so a candidate
 // costs one pair of table reads; the first match in unit order then finds its
 // lowest fitting rotation across the wave (lane r tests rotation r).
-template <int U, bool SK, bool R64, bool BT>
+template <int U, int SK, bool R64, bool BT>
 __device__ __forceinline__ uint64_t group_leaf_rot(const uint64_t *__restrict__ kp, uint32_t L, uint32_t nl,
                                                    uint64_t u0, const uint16_t *canon) {
     // BT: position (h16 * L) >> 16 of every 16-bit hash read from the byte table
@@ -920,8 +955,8 @@ __device__ __forceinline__ uint64_t group_leaf_rot(const uint64_t *__restrict__ 
 #pragma unroll
     for (int u = 0; u < U; u++) mk[u] = 0;
     if constexpr (R64) {
-        each_r64<U>(kp, 0, nl, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
-        each_r64<U>(kp, nl, L, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << (r + 16); });
+        each_r64<U, SK>(kp, 0, nl, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
+        each_r64<U, SK>(kp, nl, L, sd, L, [&](int u, uint32_t r) { mk[u] |= 1u << (r + 16); });
     } else if constexpr (BT) {
         uint32_t mr[U];
 #pragma unroll
@@ -955,7 +990,7 @@ __device__ __forceinline__ uint64_t group_leaf_rot(const uint64_t *__restrict__ 
 // Leaf without rotation (SIMDRecSplit.hpp:510-599): lowest x whose m keys land on
 // m distinct positions.  A prefix of ceil(3 sqrt(m)) keys must already be
 // collision-free; waves skip the rest when no lane passes (lossless).
-template <int U, bool SK, bool R64>
+template <int U, int SK, bool R64>
 __device__ __forceinline__ uint64_t group_leaf_brute(const uint64_t *__restrict__ kp, uint32_t m, uint32_t mid,
                                                      uint64_t u0) {
     const uint64_t S = c_start_seed[kSeedLeaf];
@@ -965,7 +1000,7 @@ __device__ __forceinline__ uint64_t group_leaf_brute(const uint64_t *__restrict_
     for (int u = 0; u < U; u++) mk[u] = 0;
     const Seeds<U> sd(u0 + S, 1);
     auto part = [&](uint32_t b, uint32_t e) {
-        if constexpr (R64) each_r64<U>(kp, b, e, sd, m, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
+        if constexpr (R64) each_r64<U, SK>(kp, b, e, sd, m, [&](int u, uint32_t r) { mk[u] |= 1u << r; });
         else each_hash<U, SK>(kp, b, e, sd, [&](int u, uint32_t h) { mk[u] |= 1u << (__umul24(h, m) >> 16); });
     };
     part(0, mid);
@@ -1052,15 +1087,15 @@ __device__ __forceinline__ uint32_t post_pos(uint32_t t, uint32_t m16) {
 
 // Calls g(pos) for every key of kp[begin, end) and this lane's own candidate at
 // base + off (off < 2^32, at most max_off over the wave).
-template <bool R64, typename G>
+template <bool R64, int SK, typename G>
 __device__ __forceinline__ void each_pos_lane(const uint64_t *__restrict__ kp, uint32_t begin, uint32_t end,
                                               uint64_t base_any, uint32_t off, uint32_t max_off, uint32_t m, G &&g) {
     const uint64_t base = uni64(base_any);
     if constexpr (R64) {
-        stream_keys_scalar(kp, begin, end, [&](uint64_t k) { g(remap64(k + base + off, m)); });
+        stream_keys_uniform<SK>(kp, begin, end, [&](uint64_t k) { g(remap64(k + base + off, m)); });
     } else {
         const uint32_t m16 = uni(m << 16), mo = uni(max_off);
-        stream_keys_scalar(kp, begin, end, [&](uint64_t k) {
+        stream_keys_uniform<SK>(kp, begin, end, [&](uint64_t k) {
             const uint64_t S = k + base;
             const uint32_t lo = (uint32_t)S, hi = (uint32_t)(S >> 32);
             if (lo <= ~mo) g(pos_of(h16_of(hash_pre32((lo + off) ^ hi)), m16));
@@ -1100,6 +1135,19 @@ struct StageKeys {
         for (int j = 0; j < 8; j++) k[j] = lo[j];
 #pragma unroll
         for (int j = 0; j < 4; j++) k[8 + j] = ((uint64_t)r[2 * j + 1] << 32) | r[2 * j];
+    }
+    // the same from LDS; the last keys repeat kp[n - 1]
+    __device__ __forceinline__ void load_lds(const uint64_t *kp, uint32_t n_any) {
+        typedef const __attribute__((address_space(3))) uint64_t *lds_keys;
+        n = uni(n_any);
+        const uint32_t lane = lane_id();
+        const uint64_t v = ((lds_keys)(uintptr_t)(uint32_t)(uintptr_t)kp)[lane < n ? lane : n - 1];
+#pragma unroll
+        for (int j = 0; j < kStageKeys; j++) {
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, j);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), j);
+            k[j] = ((uint64_t)hi << 32) | lo;
+        }
     }
 };
 
@@ -1175,7 +1223,7 @@ __device__ __forceinline__ uint64_t fit_rotation(unsigned long long cand, uint32
 // valid seed relative to the claim (candidate index, times L plus the rotation for
 // rotation leaves) or kNone.  Rotation leaves: kp[0, nl) even, kp[nl, L) odd; the
 // first stage took the first k keys of the larger half.
-template <bool ROT, bool R64>
+template <bool ROT, bool R64, int SK = kKeysScalar>
 __device__ __forceinline__ uint64_t stage_test(const uint64_t *__restrict__ kp, uint32_t m, uint32_t nl, uint32_t k,
                                                uint64_t base, uint32_t stride, uint32_t max_idx, StageQueue &sq,
                                                const uint16_t *canon) {
@@ -1188,7 +1236,7 @@ __device__ __forceinline__ uint64_t stage_test(const uint64_t *__restrict__ kp, 
     uint64_t hit = kNone;
     if constexpr (!ROT) {
         uint32_t mk = e.x;
-        each_pos_lane<R64>(kp, k, m, base, off, max_off, m, [&](uint32_t r) { mk |= 1u << r; });
+        each_pos_lane<R64, SK>(kp, k, m, base, off, max_off, m, [&](uint32_t r) { mk |= 1u << r; });
         const unsigned long long bal = __ballot(valid && mk == full);
         if (bal) hit = (uint32_t)__builtin_amdgcn_readlane((int)e.y, __ffsll((long long)bal) - 1);
     } else {
@@ -1196,8 +1244,8 @@ __device__ __forceinline__ uint64_t stage_test(const uint64_t *__restrict__ kp, 
         const uint32_t b1 = even_first ? k : nl + k, e1 = even_first ? nl : m;  // rest of the larger half
         const uint32_t b2 = even_first ? nl : 0, e2 = even_first ? m : nl;      // the other half
         uint32_t m1 = e.x, m2 = 0;
-        each_pos_lane<R64>(kp, b1, e1, base, off, max_off, m, [&](uint32_t r) { m1 |= 1u << r; });
-        each_pos_lane<R64>(kp, b2, e2, base, off, max_off, m, [&](uint32_t r) { m2 |= 1u << r; });
+        each_pos_lane<R64, SK>(kp, b1, e1, base, off, max_off, m, [&](uint32_t r) { m1 |= 1u << r; });
+        each_pos_lane<R64, SK>(kp, b2, e2, base, off, max_off, m, [&](uint32_t r) { m2 |= 1u << r; });
         const uint32_t ml = even_first ? m1 : m2, mr = even_first ? m2 : m1;
         unsigned long long cand;
         // canon (leaves of at most kNecklaceMax keys): the least rotations decide,

@@ -10,7 +10,7 @@
 // count (node lists by n, Golomb-Rice and Elias-Fano arrays by bounds checked on
 // the device), the census comes from a per-leaf table of node counts by bucket
 // size, and the search, split and encoding kernels read their counts from device
-// memory.  A build whose descriptors or Elias-Fano arrays would pass the bounds
+// memory.  Small buckets run as whole trees, as in the ordinary build.  A build whose descriptors or Elias-Fano arrays would pass the bounds
 // stops writing and reports RS_ERR_ARG; the bounds are several times the sizes
 // RecSplit reaches.
 
@@ -46,18 +46,23 @@ __global__ __launch_bounds__(256) void k_fill(T *__restrict__ p, uint64_t cap, T
 
 // Node counts per list of the whole build from the bucket-size histogram and the
 // per-size table (table[m * kNumLists + l] = nodes of list l in a bucket of m
-// keys), their prefix sums (list bases), and the oversized-bucket error.  One
-// workgroup of 256 threads.
+// keys), their prefix sums (list bases), the largest bucket below kMaxBucket, and the
+// oversized-bucket error.  One workgroup of 256 threads.
 __global__ __launch_bounds__(256) void k_plan_census(const uint32_t *__restrict__ hist,
                                                      const uint32_t *__restrict__ table, uint64_t *__restrict__ count,
-                                                     uint64_t *__restrict__ lbase, uint32_t *__restrict__ err) {
+                                                     uint64_t *__restrict__ lbase, uint32_t *__restrict__ err,
+                                                     uint32_t *__restrict__ max_bucket) {
     __shared__ uint64_t s[kNumLists][256];
+    __shared__ uint32_t s_max;
+    if (threadIdx.x == 0) s_max = 0;
+    __syncthreads();
     uint64_t acc[kNumLists];
 #pragma unroll
     for (int l = 0; l < kNumLists; l++) acc[l] = 0;
     for (uint32_t m = threadIdx.x; m < kMaxBucket; m += blockDim.x) {
         const uint64_t h = hist[m];
         if (!h) continue;
+        atomicMax(&s_max, m);
 #pragma unroll
         for (int l = 0; l < kNumLists; l++) acc[l] += h * table[m * kNumLists + l];
     }
@@ -77,6 +82,7 @@ __global__ __launch_bounds__(256) void k_plan_census(const uint32_t *__restrict_
             b += s[l][0];
         }
         if (hist[kMaxBucket]) atomicOr(err, kErrBucketTooLarge);
+        *max_bucket = s_max;
     }
 }
 
@@ -215,6 +221,7 @@ struct rs_plan {
     std::vector<double> level_nodes;     // ... and its expected nodes
     std::vector<char> mostly_full;       // ... and whether most of its nodes are of full size
     uint32_t likely_max_bucket = 0;  // bucket sizes above this are vanishingly rare
+    bool tree = false;               // buckets run as whole trees (k_tree)
     // device buffers
     KeyTile *tiles = nullptr;
     uint32_t *counts = nullptr, *size_hist = nullptr, *err = nullptr, *cursor = nullptr, *list_fill = nullptr,
@@ -240,12 +247,14 @@ namespace rsa {
 
 // Node counts per list of one bucket of each size m < kMaxBucket (the census of
 // the ordinary build, one bucket at a time), the expected key evaluations of
-// those nodes' searches, and how many of them are aggregation nodes of full size.
+// those nodes' searches and of the heaviest one, and how many of them are aggregation
+// nodes of full size.
 static std::vector<uint32_t> census_table(const SplitParams &P, bool rotate, std::vector<double> &evals,
-                                          std::vector<uint32_t> &full) {
+                                          std::vector<uint32_t> &full, std::vector<double> &most) {
     std::vector<uint32_t> t((size_t)kMaxBucket * kNumLists, 0);
     evals.assign((size_t)kMaxBucket * kNumLists, 0.0);
     full.assign((size_t)kMaxBucket * kNumLists, 0);
+    most.assign((size_t)kMaxBucket * kNumLists, 0.0);
     const Memo &memo = golomb_memo(P.leaf);
     std::vector<SubCensus> small(kMaxBucket);
     for (uint32_t m = 2; m < kMaxBucket; m++) {
@@ -255,6 +264,7 @@ static std::vector<uint32_t> census_table(const SplitParams &P, bool rotate, std
             t[(size_t)m * kNumLists + l] = (uint32_t)c.count[l];
             evals[(size_t)m * kNumLists + l] = c.evals[l];
             full[(size_t)m * kNumLists + l] = (uint32_t)c.full[l];
+            most[(size_t)m * kNumLists + l] = c.most[l];
         }
     }
     return t;
@@ -280,26 +290,63 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
         p->counts, NB, p->memo + kMaxBucket, p->counts64, p->node_cnt, p->size_hist);
     scan_level(s, p->counts, true, NB, p->acc, p->scan_tmp);
     scan_level(s, p->node_cnt, false, NB, p->node_base, p->scan_tmp);
-    k_plan_census<<<1, 256, 0, s>>>(p->size_hist, p->census, p->list_count, p->list_base, p->err);
+    k_plan_census<<<1, 256, 0, s>>>(p->size_hist, p->census, p->list_count, p->list_base, p->err, p->ctl + 2);
     k_scatter<<<p->n_tiles, 256, (size_t)priv_max * 4, s>>>(p->tiles, p->acc, p->cursor, p->sorted, priv_max);
-    // buckets up to the likely largest size with a small LDS footprint, larger
-    // ones (possible, vanishingly rare) by a second pass with room for 4096 keys
-    uint32_t sort_p = 1;
-    while (sort_p < p->likely_max_bucket) sort_p <<= 1;
-    k_sort_buckets<<<NB, p->likely_max_bucket > 512 ? 256 : 64, (size_t)sort_p * 8, s>>>(
-        p->sorted, p->acc, p->err, rotate ? p->leaf : 0, 0, p->likely_max_bucket);
-    if (p->likely_max_bucket < kMaxBucket - 1)
-        k_sort_buckets<<<NB, 256, (size_t)4096 * 8, s>>>(p->sorted, p->acc, p->err, rotate ? p->leaf : 0,
-                                                         p->likely_max_bucket + 1, kMaxBucket - 1);
-    ExpandArgs ea{P, rotate ? 1 : 0, p->pool, p->list_base, p->list_fill, p->node_m};
-    k_expand<<<(NB + 63) / 64, 64, 0, s>>>(p->acc, p->node_base, NB, ea);
+    const AggrLayout up_l = aggr_layout(P.lower, P.upper / P.lower);
+    const AggrLayout lo_l = aggr_layout(P.leaf, P.lower / P.leaf);
+    if (p->tree) {
+        // buckets up to the likely largest size with a small LDS footprint, larger
+        // ones (possible, vanishingly rare) by a second launch with room for any
+        k_fill<uint32_t><<<1, 64, 0, s>>>(p->ctl, 2, 0u);
+        TreeArgs a{};
+        a.acc = p->acc;
+        a.node_base = p->node_base;
+        a.sorted = p->sorted;
+        a.seeds = p->seeds;
+        a.node_m = p->node_m;
+        a.bits = p->bits;
+        a.evals = p->evals;
+        a.work = p->work;
+        a.memo = p->memo;
+        a.err = p->err;
+        a.ctl = p->ctl;
+        a.nb = NB;
+        a.P = P;
+        a.rotate = rotate ? 1 : 0;
+        a.max_m = p->likely_max_bucket;
+        a.cap = (p->likely_max_bucket + 7) & ~7u;
+        a.up_fb = up_l.fb;
+        a.up_magic = up_l.magic;
+        a.lo_fb = lo_l.fb;
+        a.lo_magic = lo_l.magic;
+        a.stop = p->err;
+        a.stop_mask = kErrBucketTooLarge;
+        launch_tree(s, a, r64, (uint32_t)p->num_cus);
+        a.ctl = p->ctl + 1;
+        a.min_m = p->likely_max_bucket + 1;
+        a.max_m = kMaxBucket - 1;
+        a.cap = kMaxBucket;
+        a.max_bucket = p->ctl + 2;
+        launch_tree(s, a, r64, (uint32_t)p->num_cus);
+    } else {
+        // buckets up to the likely largest size with a small LDS footprint, larger
+        // ones (possible, vanishingly rare) by a second pass with room for 4096 keys
+        uint32_t sort_p = 1;
+        while (sort_p < p->likely_max_bucket) sort_p <<= 1;
+        k_sort_buckets<<<NB, p->likely_max_bucket > 512 ? 256 : 64, (size_t)sort_p * 8, s>>>(
+            p->sorted, p->acc, p->err, rotate ? p->leaf : 0, 0, p->likely_max_bucket);
+        if (p->likely_max_bucket < kMaxBucket - 1)
+            k_sort_buckets<<<NB, 256, (size_t)4096 * 8, s>>>(p->sorted, p->acc, p->err, rotate ? p->leaf : 0,
+                                                             p->likely_max_bucket + 1, kMaxBucket - 1);
+        ExpandArgs ea{P, rotate ? 1 : 0, p->pool, p->list_base, p->list_fill, p->node_m};
+        k_expand<<<(NB + 63) / 64, 64, 0, s>>>(p->acc, p->node_base, NB, ea);
+        HIP_CHECK(hipGetLastError());
+    }
     HIP_CHECK(hipGetLastError());
 
     // ---- search levels, sizes from the device census
-    const AggrLayout up_l = aggr_layout(P.lower, P.upper / P.lower);
-    const AggrLayout lo_l = aggr_layout(P.leaf, P.lower / P.leaf);
     const Tune &tn = p->tune;
-    for (size_t li = 0; li < p->lists.size(); li++) {
+    for (size_t li = 0; li < p->lists.size() && !p->tree; li++) {
         const int l = p->lists[li];
         // levels only buckets far above the likely largest size reach run on a
         // small grid: correct if such a bucket appears, nearly free when none does
@@ -364,8 +411,9 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
     // ---- encoding (the ordinary build's steps 5-7 for one set)
     const uint32_t *memo = p->memo;
     EncodeArgs ca{p->acc, p->node_base, p->seeds, p->node_m, memo, memo + kMaxBucket, NB, P, rotate ? 1 : 0, p->err};
-    k_bucket_bits<<<(uint32_t)std::min<uint64_t>((NB + 3) / 4, (uint64_t)p->num_cus * 8), 256, 0, s>>>(
-        ca, p->bits, p->evals);
+    if (!p->tree)
+        k_bucket_bits<<<(uint32_t)std::min<uint64_t>((NB + 3) / 4, (uint64_t)p->num_cus * 8), 256, 0, s>>>(
+            ca, p->bits, p->evals);
     scan_level(s, p->bits, false, NB, p->pos, p->scan_tmp);
     k_plan_rice<<<1, 64, 0, s>>>(p->pos, NB, p->cap_rice, p->enc, p->meta, p->err);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->rice, p->cap_rice, 0ull, &p->meta->rice_words, 2);
@@ -405,7 +453,6 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
         p->n_tiles = (uint32_t)((n + kTileKeys - 1) / kTileKeys);
         const uint64_t NB = p->nb;
         const SplitParams P = split_params(leaf);
-        (void)P;
         // bounds: nodes < n (a tree over m keys has at most m - 1 nodes); descriptors
         // at most 8 bits per key plus a word per bucket (RecSplit stores ~1.6);
         // Elias-Fano lower bits at most 128 per bucket, upper bits at most 3 per bucket
@@ -464,9 +511,9 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
         real.size = p->mem_bytes;
         plan_layout(real);
         // tables, and the tree levels some bucket size can reach
-        std::vector<double> evals;
+        std::vector<double> evals, most;
         std::vector<uint32_t> full;
-        const std::vector<uint32_t> table = census_table(split_params(leaf), (flags & kFlagRotate) != 0, evals, full);
+        const std::vector<uint32_t> table = census_table(split_params(leaf), (flags & kFlagRotate) != 0, evals, full, most);
         HIP_CHECK(hipMemcpy(p->memo, golomb_memo(leaf).data(), sizeof(uint32_t) * kMaxBucket, hipMemcpyHostToDevice));
         HIP_CHECK(hipMemcpy(p->memo + kMaxBucket, tree_nodes(leaf).data(), sizeof(uint32_t) * kMaxBucket,
                             hipMemcpyHostToDevice));
@@ -480,9 +527,10 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
         std::vector<double> pmf(kMaxBucket, 0.0);
         for (uint32_t m = 0; m < kMaxBucket; m++)
             pmf[m] = std::exp((double)m * std::log(mean) - mean - std::lgamma((double)m + 1.0));
+        TreeWork tw;
         for (int l = 0; l < kNumLists; l++) {
             bool any = false, lik = false;
-            double e = 0, cnt = 0, nfull = 0;
+            double e = 0, cnt = 0, nfull = 0, mx = 0;
             for (uint32_t m = 2; m < kMaxBucket; m++)
                 if (table[(size_t)m * kNumLists + l]) {
                     any = true;
@@ -490,7 +538,9 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
                     e += pmf[m] * evals[(size_t)m * kNumLists + l];
                     cnt += pmf[m] * table[(size_t)m * kNumLists + l];
                     nfull += pmf[m] * full[(size_t)m * kNumLists + l];
+                    if (pmf[m] * (double)NB > 0.01) mx = std::max(mx, most[(size_t)m * kNumLists + l]);
                 }
+            tw.add(e * (double)NB, cnt * (double)NB, mx);
             if (any) {
                 p->lists.push_back(l);
                 p->likely.push_back(lik ? 1 : 0);
@@ -499,6 +549,8 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
                 p->mostly_full.push_back(2 * nfull >= cnt ? 1 : 0);
             }
         }
+        p->tree = tree_fits(p->tune, aggr_layout(P.lower, P.upper / P.lower), aggr_layout(P.leaf, P.lower / P.leaf),
+                            p->likely_max_bucket, tw, (double)NB, (uint32_t)p->num_cus);
     });
     if (rc != RS_OK) {
         if (p->mem) (void)hipFree(p->mem);

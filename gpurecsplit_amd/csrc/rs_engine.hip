@@ -121,13 +121,28 @@ struct HostBuf {
     }
 };
 
-// Device-resident copy of a structure for batched queries; word counts are the
-// readable words of each array.
+// Device-resident copy of a structure for batched queries, in one allocation; word
+// counts are the readable words of each array.
 struct DeviceCopy {
     int device = 0;
+    uint64_t *mem = nullptr;
     uint64_t *rice = nullptr, *lower = nullptr, *upper_c = nullptr, *upper_p = nullptr, *jump = nullptr;
     uint32_t *memo = nullptr;
     uint64_t n_rice = 0, n_lower = 0, n_uc = 0, n_up = 0, n_jump = 0;
+    // The arrays one after another from p on; the memo table at m.
+    void place(uint64_t *p, uint64_t rice_words, const std::array<uint64_t, 4> &ef_words, uint32_t *m) {
+        n_rice = rice_words;
+        n_lower = ef_words[0];
+        n_uc = ef_words[1];
+        n_up = ef_words[2];
+        n_jump = ef_words[3];
+        rice = p;
+        lower = rice + n_rice;
+        upper_c = lower + n_lower;
+        upper_p = upper_c + n_uc;
+        jump = upper_p + n_up;
+        memo = m;
+    }
 };
 
 void device_copy_free(DeviceCopy *d) {
@@ -135,9 +150,7 @@ void device_copy_free(DeviceCopy *d) {
     int prev = 0;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(d->device);
-    for (void *p : {(void *)d->rice, (void *)d->lower, (void *)d->upper_c, (void *)d->upper_p, (void *)d->jump,
-                    (void *)d->memo})
-        if (p) (void)hipFree(p);
+    if (d->mem) (void)hipFree(d->mem);
     (void)hipSetDevice(prev);
     delete d;
 }
@@ -405,9 +418,10 @@ struct rs_ctx {
     int num_cus = 0;
     hipStream_t stream = nullptr;
     std::mutex mu;
-    DevBuf keys_in, counts, counts64, cursor, acc, node_cnt, node_base, size_hist, scan_tmp, sorted, pool, list_base,
-        list_fill, node_m, seeds, state, running, ctl, err, bits, pos, evals, work, rice, ef_scalars, ef_lower, ef_uc,
-        ef_up, ef_jump, tiles, set_idx, set_gather, set_enc, bit_off, clock, str_bytes, str_off, tune_keys, wave_clock;
+    // counts: report words, size histogram, bucket counts and cursors; rice: every result word
+    DevBuf keys_in, counts, counts64, acc, node_cnt, node_base, scan_tmp, sorted, pool, list_base, list_fill, node_m,
+        seeds, state, running, bits, pos, rice, ef_scalars, tiles, set_idx, set_enc, bit_off, clock, str_bytes, str_off,
+        tune_keys, wave_clock;
     double time_limit_s = 0;  // 0: none
     bool wave_times = false;  // RS_WAVE_TIMES: record search waves' start and exit times
     int wall_khz = 0;         // device wall-clock rate
@@ -676,13 +690,34 @@ static uint32_t launch_tree(hipStream_t s, TreeArgs a, bool r64, uint32_t num_cu
     return blocks * wpg;
 }
 
-__global__ void k_gather_u64(const uint64_t *__restrict__ src, const uint64_t *__restrict__ idx, uint64_t n,
-                             uint64_t *__restrict__ out) {
+// What the host reads after the search, in one block beside the counters: the used
+// seed slots and the bit position of every set's first bucket (idx, nullptr: one set of
+// nb buckets) and of the end.
+__global__ __launch_bounds__(256) void k_report(const uint64_t *__restrict__ pos, const uint64_t *__restrict__ slots,
+                                                const uint64_t *__restrict__ idx, uint64_t nb, uint64_t n,
+                                                uint64_t *__restrict__ out_slots, uint64_t *__restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = src[idx[i]];
+    if (i < n) out[i] = pos[idx ? idx[i] : i * nb];
+    if (i == 0) *out_slots = *slots;
+}
+
+// Workgroups per set of the encoding kernels that run (set, part) workgroups: about
+// 1024 buckets each, up to 32768 workgroups in all.
+static uint32_t ef_parts(uint64_t max_nb, uint64_t sets) {
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({(max_nb + 1023) / 1024, 256, 32768 / std::max<uint64_t>(sets, 1)}));
 }
 
 constexpr uint64_t kTileKeys = 1 << 14;  // keys per histogram / scatter workgroup
+
+// Keys per tile of a build of n keys whose largest set has max_nb buckets.  Larger
+// tiles when there are keys for two per CU: fewer global atomics per key.  Small
+// builds take tiles for two per CU, but of at least twice the buckets (every tile
+// adds its touched buckets to the global counts) and 2048 keys: 100K keys in 1,000
+// buckets 20.8 -> 5.6 us (histogram), 29.2 -> 9.8 us (scatter).
+static uint64_t tile_size(uint64_t n, uint64_t max_nb, uint32_t num_cus) {
+    if (n >= 8 * kTileKeys * num_cus) return 4 * kTileKeys;
+    return std::min(kTileKeys, std::max<uint64_t>({2048, 2 * max_nb, n / (2 * (uint64_t)num_cus)}));
+}
 
 static std::string autotune(rs_ctx *c, uint32_t leaf, uint64_t bucket, int flags, uint64_t sample_keys);
 
@@ -767,14 +802,16 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     std::vector<uint64_t> nbs(S), bbase(S + 1);
     std::vector<KeyTile> tiles;
     uint64_t NB = 0, max_nb = 0;
-    // larger tiles when there are keys for two per CU: fewer global atomics per key
-    const uint64_t tile_keys = set_off[S] - set_off[0] >= 8 * kTileKeys * (uint64_t)c->num_cus ? 4 * kTileKeys : kTileKeys;
     for (size_t i = 0; i < S; i++) {
         const uint64_t n = set_off[i + 1] - set_off[i];
         nbs[i] = std::max<uint64_t>(1, (n + bucket_size - 1) / bucket_size);
+        max_nb = std::max(max_nb, nbs[i]);
+    }
+    const uint64_t tile_keys = tile_size(set_off[S] - set_off[0], max_nb, (uint32_t)c->num_cus);
+    for (size_t i = 0; i < S; i++) {
+        const uint64_t n = set_off[i + 1] - set_off[i];
         bbase[i] = NB;
         NB += nbs[i];
-        max_nb = std::max(max_nb, nbs[i]);
         for (uint64_t k = 0; k < n; k += tile_keys)
             tiles.push_back(KeyTile{set_keys[i], k, std::min(k + tile_keys, n), nbs[i], bbase[i]});
     }
@@ -794,17 +831,30 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     // ---- 1. bucket histogram and per-bucket metadata
     const int e_part0 = ev_record(c);
     KeyTile *d_tiles = c->tiles.get<KeyTile>(tiles.size());
-    HIP_CHECK(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(KeyTile), hipMemcpyHostToDevice, s));
-    uint32_t *counts = c->counts.get<uint32_t>(NB);
+    const void *tile_src = tiles.data();
+    if (tiles.size() * sizeof(KeyTile) <= 16384) {  // through pinned staging
+        memcpy((uint8_t *)c->h_pinned + 32768, tiles.data(), tiles.size() * sizeof(KeyTile));
+        tile_src = (uint8_t *)c->h_pinned + 32768;
+    }
+    HIP_CHECK(hipMemcpyAsync(d_tiles, tile_src, tiles.size() * sizeof(KeyTile), hipMemcpyHostToDevice, s));
+    // everything that starts at zero, in one block (one fill): the words the host reads
+    // after the search (report), then the size histogram, the bucket counts and cursors
+    constexpr uint64_t kErrWord = 0, kCtlWord = 2, kEvalWord = 10, kWorkWord = kEvalWord + 2 * kNumKinds,
+                       kSlotWord = kWorkWord + kNumLists, kPosWord = kSlotWord + 1;
+    const uint64_t report_words = kPosWord + S + 1, hist_words = (kMaxBucket + 2) / 2, bucket_words = (NB + 1) / 2;
+    uint64_t *report = c->counts.get<uint64_t>(report_words + hist_words + 2 * bucket_words);
+    HIP_CHECK(hipMemsetAsync(report, 0, 8 * (report_words + hist_words + 2 * bucket_words), s));
+    uint32_t *err = (uint32_t *)(report + kErrWord);
+    uint32_t *ctl = (uint32_t *)(report + kCtlWord);
+    unsigned long long *evals = (unsigned long long *)report + kEvalWord;  // evaluations, then seeds
+    unsigned long long *work = (unsigned long long *)report + kWorkWord;
+    uint32_t *size_hist = (uint32_t *)(report + report_words);
+    uint32_t *counts = (uint32_t *)(report + report_words + hist_words);
+    uint32_t *cursor = (uint32_t *)(report + report_words + hist_words + bucket_words);
     uint64_t *counts64 = c->counts64.get<uint64_t>(NB);
     uint64_t *acc = c->acc.get<uint64_t>(NB + 1);
     uint64_t *node_cnt = c->node_cnt.get<uint64_t>(NB);
     uint64_t *node_base = c->node_base.get<uint64_t>(NB + 1);
-    uint32_t *size_hist = c->size_hist.get<uint32_t>(kMaxBucket + 1);
-    uint32_t *err = c->err.get<uint32_t>(4);
-    HIP_CHECK(hipMemsetAsync(counts, 0, NB * 4, s));
-    HIP_CHECK(hipMemsetAsync(size_hist, 0, (kMaxBucket + 1) * 4, s));
-    HIP_CHECK(hipMemsetAsync(err, 0, 16, s));
     const uint32_t priv_max = (uint32_t)std::min<uint64_t>(max_nb, 16384);
     k_bucket_hist<<<tiles.size(), 256, (size_t)priv_max * 4, s>>>(d_tiles, counts, priv_max);
     HIP_CHECK(hipGetLastError());
@@ -838,8 +888,6 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
 
     // ---- 2. scatter and per-bucket sort
     uint64_t *sorted = c->sorted.get<uint64_t>(n_total + 8);  // +8: look-ahead loads of the search
-    uint32_t *cursor = c->cursor.get<uint32_t>(NB);
-    HIP_CHECK(hipMemsetAsync(cursor, 0, NB * 4, s));
     k_scatter<<<tiles.size(), 256, (size_t)priv_max * 4, s>>>(d_tiles, acc, cursor, sorted, priv_max);
     HIP_CHECK(hipGetLastError());
     const Tune tn = tune_for(c, leaf);
@@ -893,25 +941,19 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     const uint32_t n_waves = blocks * 4;
     st.search_waves = n_waves;
     int *running = c->running.get<int>(n_waves);
-    uint32_t *ctl = c->ctl.get<uint32_t>(16);
-    unsigned long long *work = c->work.get<unsigned long long>(kNumLists);
-    HIP_CHECK(hipMemsetAsync(work, 0, kNumLists * 8, s));
     unsigned long long *wave_clock = nullptr;
     if (c->wave_times && !t_arena) {
         wave_clock = c->wave_clock.get<unsigned long long>((size_t)kNumLists * 2 * n_waves);
         HIP_CHECK(hipMemsetAsync(wave_clock, 0, (size_t)kNumLists * 2 * n_waves * 8, s));
     }
     uint64_t *bits = c->bits.get<uint64_t>(NB);
-    unsigned long long *evals = c->evals.get<unsigned long long>(2 * kNumKinds);  // evaluations, then seeds
-    HIP_CHECK(hipMemsetAsync(evals, 0, 2 * kNumKinds * 8, s));
     struct PhaseEvents {
         uint32_t kind;
         int search0, search1, split1;
     };
     std::vector<PhaseEvents> phase_ev;
     if (tree) {
-        // the whole trees, one wave per bucket; work counters by kind in work[0, kNumKinds)
-        HIP_CHECK(hipMemsetAsync(ctl, 0, 64, s));
+        // the whole trees; work counters by kind in work[0, kNumKinds)
         TreeArgs a{};
         a.acc = acc;
         a.node_base = node_base;
@@ -1019,34 +1061,37 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         HIP_CHECK(hipGetLastError());
     }
     scan_u64(c, bits, false, NB, pos);
-    uint64_t *d_bidx = c->set_idx.get<uint64_t>(S + 1);
-    uint64_t *d_gath = c->set_gather.get<uint64_t>(S + 1);
-    HIP_CHECK(hipMemcpyAsync(d_bidx, bbase.data(), (S + 1) * 8, hipMemcpyHostToDevice, s));
-    k_gather_u64<<<(S + 1 + 255) / 256, 256, 0, s>>>(pos, d_bidx, S + 1, d_gath);
-    HIP_CHECK(hipGetLastError());
-    std::vector<uint64_t> pos_at(S + 1);
-    uint64_t *h64 = (uint64_t *)c->h_pinned;
-    HIP_CHECK(hipMemcpyAsync(pos_at.data(), d_gath, (S + 1) * 8, hipMemcpyDeviceToHost, s));
-    // pinned staging: error flags at byte 64, work counters at 128..296, evaluations
-    // and seeds at 512..592
-    HIP_CHECK(hipMemcpyAsync(h64 + 64, evals, 2 * kNumKinds * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h64 + 16, work, kNumLists * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h + 16, err, 4, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h64 + 80, node_base + NB, 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (h[16] & kErrTimeout)
-        throw BuildError(RS_ERR_TIMEOUT, "the build passed the context's time limit during the seed search");
-    if (tree) check_partition(h[16], h64[80]);
-    for (int k = 0; k < kNumKinds; k++) {
-        st.evals[k] = h64[64 + k];
-        st.seeds[k] = h64[64 + kNumKinds + k];
+    uint64_t *d_bidx = nullptr;
+    if (S > 1) {
+        d_bidx = c->set_idx.get<uint64_t>(S + 1);
+        HIP_CHECK(hipMemcpyAsync(d_bidx, bbase.data(), (S + 1) * 8, hipMemcpyHostToDevice, s));
     }
-    static_assert(16 + kNumLists <= 64, "work counters overlap the evaluation counts");
+    k_report<<<(S + 1 + 255) / 256, 256, 0, s>>>(pos, node_base + NB, d_bidx, NB, S + 1, report + kSlotWord,
+                                                 report + kPosWord);
+    HIP_CHECK(hipGetLastError());
+    // into pinned memory where it fits (32 KiB of the staging area)
+    std::vector<uint64_t> report_copy;
+    uint64_t *hr = (uint64_t *)c->h_pinned;
+    if (report_words > 4096) {
+        report_copy.resize(report_words);
+        hr = report_copy.data();
+    }
+    HIP_CHECK(hipMemcpyAsync(hr, report, report_words * 8, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+    const uint32_t err_word = (uint32_t)hr[kErrWord];
+    const uint64_t *pos_at = hr + kPosWord;
+    if (err_word & kErrTimeout)
+        throw BuildError(RS_ERR_TIMEOUT, "the build passed the context's time limit during the seed search");
+    if (tree) check_partition(err_word, hr[kSlotWord]);
+    for (int k = 0; k < kNumKinds; k++) {
+        st.evals[k] = hr[kEvalWord + k];
+        st.seeds[k] = hr[kEvalWord + kNumKinds + k];
+    }
     for (int l = 0; l < kNumLists && !tree; l++)
-        st.executed_evals[l < (int)kMaxDepth ? kHigher : l - kMaxDepth + 1] += h64[16 + l];
-    for (int k = 0; k < kNumKinds && tree; k++) st.executed_evals[k] = h64[16 + k];
+        st.executed_evals[l < (int)kMaxDepth ? kHigher : l - kMaxDepth + 1] += hr[kWorkWord + l];
+    for (int k = 0; k < kNumKinds && tree; k++) st.executed_evals[k] = hr[kWorkWord + k];
     if (wave_clock) wave_time_stats(c, wave_clock, n_waves, cen.count, st);
-    if (h[16] & 2) throw BuildError(RS_ERR_SEED_OVERFLOW, "a node search passed the 2^44 seed limit");
+    if (err_word & kErrSeedLimit) throw BuildError(RS_ERR_SEED_OVERFLOW, "a node search passed the 2^44 seed limit");
 
     // ---- 6. Golomb-Rice: per-set vectors packed one after another
     std::vector<SetEnc> enc(S);
@@ -1061,18 +1106,40 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         rice_total += rice_words[i];
         st.rice_bits += B;
     }
+    // One buffer of result words, cleared at once: a status word (the fill kernel's
+    // errors), every set's descriptors, then the Elias-Fano arrays, whose exact sizes
+    // follow from the scalars: at most 2 lower words per bucket (two widths below 64)
+    // and 3 bits per bucket in either upper array (u >> l < 2 (nb + 1)).
+    uint64_t ef_cap = 0;
+    for (size_t i = 0; i < S; i++) ef_cap += 2 * (nbs[i] + 2) + 2 * (3 * (nbs[i] + 1) / 64 + 2) + ef_jump_words(nbs[i]);
+    unsigned long long *result = c->rice.get<unsigned long long>(1 + rice_total + ef_cap);
+    HIP_CHECK(hipMemsetAsync(result, 0, (1 + rice_total + ef_cap) * 8, s));
+    unsigned long long *rice = result + 1;
     SetEnc *d_enc = c->set_enc.get<SetEnc>(S);
-    HIP_CHECK(hipMemcpyAsync(d_enc, enc.data(), S * sizeof(SetEnc), hipMemcpyHostToDevice, s));
-    unsigned long long *rice = c->rice.get<unsigned long long>(rice_total + 2);
+    // small uploads go through the pinned staging area's second half
+    auto upload_enc = [&]() {
+        const void *src = enc.data();
+        if (S * sizeof(SetEnc) <= 16384) {
+            memcpy((uint8_t *)c->h_pinned + 49152, enc.data(), S * sizeof(SetEnc));
+            src = (uint8_t *)c->h_pinned + 49152;
+        }
+        HIP_CHECK(hipMemcpyAsync(d_enc, src, S * sizeof(SetEnc), hipMemcpyHostToDevice, s));
+    };
+    upload_enc();
     long long *bit_off = c->bit_off.get<long long>(NB);
-    HIP_CHECK(hipMemsetAsync(rice, 0, (rice_total + 2) * 8, s));
-    k_set_offsets<<<S, 256, 0, s>>>(d_enc, pos, bit_off, rice);
-    k_rice_write<<<(NB + 3) / 4, 256, 0, s>>>(ca, pos, bit_off, rice);
     EfScalars *d_efs = c->ef_scalars.get<EfScalars>(S);
-    k_ef_scalars<<<S, 256, 0, s>>>(d_enc, acc, pos, d_efs);
+    const dim3 parts((uint32_t)S, ef_parts(max_nb, S));
+    k_set_offsets<<<parts, 256, 0, s>>>(d_enc, pos, bit_off, rice, d_efs);
+    k_rice_write<<<(NB + 3) / 4, 256, 0, s>>>(ca, pos, bit_off, rice);
+    k_ef_scalars<<<parts, 256, 0, s>>>(d_enc, acc, pos, d_efs);
     HIP_CHECK(hipGetLastError());
-    std::vector<EfScalars> he(S);
-    HIP_CHECK(hipMemcpyAsync(he.data(), d_efs, S * sizeof(EfScalars), hipMemcpyDeviceToHost, s));
+    std::vector<EfScalars> he_copy;
+    EfScalars *he = (EfScalars *)c->h_pinned;
+    if (S * sizeof(EfScalars) > 32768) {
+        he_copy.resize(S);
+        he = he_copy.data();
+    }
+    HIP_CHECK(hipMemcpyAsync(he, d_efs, S * sizeof(EfScalars), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
 
     // ---- 7. Elias-Fano: per-set widths and sizes (DoubleEF.hpp:181-202)
@@ -1106,16 +1173,12 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         tot_up += ef_words[i][2];
         tot_jump += ef_words[i][3];
     }
-    HIP_CHECK(hipMemcpyAsync(d_enc, enc.data(), S * sizeof(SetEnc), hipMemcpyHostToDevice, s));
-    unsigned long long *d_lower = c->ef_lower.get<unsigned long long>(tot_lower + 1);
-    unsigned long long *d_uc = c->ef_uc.get<unsigned long long>(tot_uc + 1);
-    unsigned long long *d_up = c->ef_up.get<unsigned long long>(tot_up + 1);
-    uint8_t *d_jump = c->ef_jump.get<uint8_t>(tot_jump * 8 + 8);
-    HIP_CHECK(hipMemsetAsync(d_lower, 0, (tot_lower + 1) * 8, s));
-    HIP_CHECK(hipMemsetAsync(d_uc, 0, (tot_uc + 1) * 8, s));
-    HIP_CHECK(hipMemsetAsync(d_up, 0, (tot_up + 1) * 8, s));
-    HIP_CHECK(hipMemsetAsync(d_jump, 0, tot_jump * 8 + 8, s));
-    k_ef_fill<<<S, 256, 0, s>>>(d_enc, d_efs, acc, pos, d_lower, d_uc, d_up, d_jump, err);
+    upload_enc();
+    if (tot_lower + tot_uc + tot_up + tot_jump > ef_cap)
+        throw BuildError(RS_ERR_INTERNAL, "Elias-Fano arrays beyond their bound");
+    unsigned long long *d_lower = rice + rice_total, *d_uc = d_lower + tot_lower, *d_up = d_uc + tot_uc;
+    uint8_t *d_jump = (uint8_t *)(d_up + tot_up);
+    k_ef_fill<<<parts, 256, 0, s>>>(d_enc, d_efs, acc, pos, d_lower, d_uc, d_up, d_jump, (uint32_t *)result);
     HIP_CHECK(hipGetLastError());
     const int e_enc_end = ev_record(c);
 
@@ -1154,47 +1217,30 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         vec(d_uc, tot_uc);
         vec(d_up, tot_up);
         vec(d_jump, tot_jump);
-        HIP_CHECK(hipMemcpyAsync(h + 16, err, 4, hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipMemcpyAsync(h, result, 4, hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipStreamSynchronize(s));
-        if (h[16] & 4) throw BuildError(RS_ERR_EF_OVERFLOW, "Elias-Fano jump offset does not fit 16 bits");
+        if (h[0] & kErrEfJump) throw BuildError(RS_ERR_EF_OVERFLOW, "Elias-Fano jump offset does not fit 16 bits");
         return {};
     }
-    // One copy per array, all sets at once, into the context's pinned staging (a
-    // copy into fresh pageable memory took 27 ms longer for the 126 MB of 4096
-    // sets of 590M keys); the handles take their words from there.
-    uint64_t *h_rice = c->h_result.get(8 * (rice_total + tot_lower + tot_uc + tot_up + tot_jump + 5));
-    uint64_t *h_lower = h_rice + rice_total + 1, *h_uc = h_lower + tot_lower + 1, *h_up = h_uc + tot_uc + 1,
-             *h_jump = h_up + tot_up + 1;
-    HIP_CHECK(hipMemcpyAsync(h_rice, rice, rice_total * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h_lower, d_lower, tot_lower * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h_uc, d_uc, tot_uc * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h_up, d_up, tot_up * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h_jump, d_jump, tot_jump * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h + 16, err, 4, hipMemcpyDeviceToHost, s));
+    // One copy of all arrays of all sets into the context's pinned staging (a copy into
+    // fresh pageable memory took 27 ms longer for the 126 MB of 4096 sets of 590M
+    // keys); the handles take their words from there.
+    const uint64_t total_words = 1 + rice_total + tot_lower + tot_uc + tot_up + tot_jump;
+    const uint64_t *h_result = c->h_result.get(8 * total_words);
+    const uint64_t *h_rice = h_result + 1, *h_lower = h_rice + rice_total, *h_uc = h_lower + tot_lower,
+                   *h_up = h_uc + tot_uc, *h_jump = h_up + tot_up;
+    HIP_CHECK(hipMemcpyAsync((void *)h_result, result, total_words * 8, hipMemcpyDeviceToHost, s));
     DeviceCopy *dc = nullptr;
     if (device_copy && S == 1) {
         dc = new DeviceCopy();
         dc->device = c->device;
-        dc->n_rice = rice_total;
-        dc->n_lower = ef_words[0][0];
-        dc->n_uc = ef_words[0][1];
-        dc->n_up = ef_words[0][2];
-        dc->n_jump = ef_words[0][3];
-        HIP_CHECK(hipMalloc(&dc->rice, (rice_total + 2) * 8));
-        HIP_CHECK(hipMalloc(&dc->lower, (dc->n_lower + 1) * 8));
-        HIP_CHECK(hipMalloc(&dc->upper_c, (dc->n_uc + 1) * 8));
-        HIP_CHECK(hipMalloc(&dc->upper_p, (dc->n_up + 1) * 8));
-        HIP_CHECK(hipMalloc(&dc->jump, dc->n_jump * 8 + 8));
-        HIP_CHECK(hipMalloc(&dc->memo, kMaxBucket * 4));
-        HIP_CHECK(hipMemcpyAsync(dc->rice, rice, (rice_total + 2) * 8, hipMemcpyDeviceToDevice, s));
-        HIP_CHECK(hipMemcpyAsync(dc->lower, d_lower, (dc->n_lower + 1) * 8, hipMemcpyDeviceToDevice, s));
-        HIP_CHECK(hipMemcpyAsync(dc->upper_c, d_uc, (dc->n_uc + 1) * 8, hipMemcpyDeviceToDevice, s));
-        HIP_CHECK(hipMemcpyAsync(dc->upper_p, d_up, (dc->n_up + 1) * 8, hipMemcpyDeviceToDevice, s));
-        HIP_CHECK(hipMemcpyAsync(dc->jump, d_jump, dc->n_jump * 8 + 8, hipMemcpyDeviceToDevice, s));
+        HIP_CHECK(hipMalloc(&dc->mem, total_words * 8 + kMaxBucket * 4));
+        dc->place(dc->mem + 1, rice_total, ef_words[0], (uint32_t *)(dc->mem + total_words));
+        HIP_CHECK(hipMemcpyAsync(dc->mem, result, total_words * 8, hipMemcpyDeviceToDevice, s));
         HIP_CHECK(hipMemcpyAsync(dc->memo, memo, kMaxBucket * 4, hipMemcpyDeviceToDevice, s));
     }
     HIP_CHECK(hipStreamSynchronize(s));
-    if (h[16] & 4) {
+    if (*(const uint32_t *)h_result & kErrEfJump) {
         if (dc) device_copy_free(dc);
         throw BuildError(RS_ERR_EF_OVERFLOW, "Elias-Fano jump offset does not fit 16 bits");
     }
@@ -1278,11 +1324,10 @@ static rs_mphf *build(rs_ctx *c, const uint64_t *d_keys, uint64_t n, uint32_t le
 
 // Every reusable device buffer of a context.
 static std::vector<DevBuf *> ctx_bufs(rs_ctx *c) {
-    return {&c->keys_in, &c->counts, &c->counts64, &c->cursor, &c->acc, &c->node_cnt, &c->node_base,
-            &c->size_hist, &c->scan_tmp, &c->sorted, &c->pool, &c->list_base, &c->list_fill, &c->node_m,
-            &c->seeds, &c->state, &c->running, &c->ctl, &c->err, &c->bits, &c->pos, &c->evals, &c->work, &c->rice,
-            &c->ef_scalars, &c->ef_lower, &c->ef_uc, &c->ef_up, &c->ef_jump, &c->tiles, &c->set_idx,
-            &c->set_gather, &c->set_enc, &c->bit_off, &c->clock, &c->str_bytes, &c->str_off, &c->tune_keys};
+    return {&c->keys_in, &c->counts, &c->counts64, &c->acc, &c->node_cnt, &c->node_base, &c->scan_tmp, &c->sorted,
+            &c->pool, &c->list_base, &c->list_fill, &c->node_m, &c->seeds, &c->state, &c->running, &c->bits, &c->pos,
+            &c->rice, &c->ef_scalars, &c->tiles, &c->set_idx, &c->set_enc, &c->bit_off, &c->clock, &c->str_bytes,
+            &c->str_off, &c->tune_keys};
 }
 
 // SplitMix64 keys on the device (the generator of the synthetic workloads): key i
@@ -1432,30 +1477,25 @@ static const DeviceCopy *device_copy_of(rs_ctx *c, rs_mphf *h) {
     DeviceCopy *dc = new DeviceCopy();
     dc->device = c->device;
     const EliasFano &ef = h->ef;
-    auto up = [&](uint64_t **dst, const uint64_t *src, uint64_t words) {
-        // one zero word of padding beyond the readable words
-        HIP_CHECK(hipMalloc(dst, (words + 1) * 8));
-        HIP_CHECK(hipMemsetAsync(*dst, 0, (words + 1) * 8, c->stream));
-        if (words) HIP_CHECK(hipMemcpyAsync(*dst, src, words * 8, hipMemcpyHostToDevice, c->stream));
+    auto up = [&](uint64_t *dst, const uint64_t *src, uint64_t words) {
+        if (words) HIP_CHECK(hipMemcpyAsync(dst, src, words * 8, hipMemcpyHostToDevice, c->stream));
     };
     try {
-        up(&dc->rice, h->rice.data(), h->rice_words);
-        up(&dc->lower, ef.lower_bits.data(), ef.lower_bits.size());
-        up(&dc->upper_c, ef.upper_cum.data(), ef.upper_cum.size());
-        up(&dc->upper_p, ef.upper_pos.data(), ef.upper_pos.size());
-        up(&dc->jump, ef.jump.data(), ef.jump.size());
-        HIP_CHECK(hipMalloc(&dc->memo, kMaxBucket * 4));
+        const uint64_t words = h->rice_words + ef.lower_bits.size() + ef.upper_cum.size() + ef.upper_pos.size() + ef.jump.size();
+        HIP_CHECK(hipMalloc(&dc->mem, words * 8 + kMaxBucket * 4));
+        dc->place(dc->mem, h->rice_words, {ef.lower_bits.size(), ef.upper_cum.size(), ef.upper_pos.size(), ef.jump.size()},
+                  (uint32_t *)(dc->mem + words));
+        up(dc->rice, h->rice.data(), dc->n_rice);
+        up(dc->lower, ef.lower_bits.data(), dc->n_lower);
+        up(dc->upper_c, ef.upper_cum.data(), dc->n_uc);
+        up(dc->upper_p, ef.upper_pos.data(), dc->n_up);
+        up(dc->jump, ef.jump.data(), dc->n_jump);
         HIP_CHECK(hipMemcpyAsync(dc->memo, h->memo->data(), kMaxBucket * 4, hipMemcpyHostToDevice, c->stream));
         HIP_CHECK(hipStreamSynchronize(c->stream));
     } catch (...) {
         device_copy_free(dc);
         throw;
     }
-    dc->n_rice = h->rice_words;
-    dc->n_lower = ef.lower_bits.size();
-    dc->n_uc = ef.upper_cum.size();
-    dc->n_up = ef.upper_pos.size();
-    dc->n_jump = ef.jump.size();
     h->dev = dc;
     return dc;
 }

@@ -1981,33 +1981,39 @@ struct SetEnc {
     uint64_t lc, lp;             // EF lower-bit widths
 };
 
-// One workgroup per set: bit offset of every bucket of the set inside the global
-// Golomb-Rice buffer, and the sentinel bit after the set's last bucket
-// (appendFixed(1, 1), SIMDRecSplit.hpp:810).
-__global__ __launch_bounds__(256) void k_set_offsets(const SetEnc *__restrict__ sets, const uint64_t *__restrict__ pos,
-                                                     long long *__restrict__ bit_off,
-                                                     unsigned long long *__restrict__ words,
-                                                     const uint32_t *__restrict__ stop = nullptr) {
-    if (stop && (*stop & kErrStopEncode)) return;
-    const SetEnc e = sets[blockIdx.x];
-    const long long off = (long long)(e.rice_word * 64) - (long long)pos[e.bbase];
-    for (uint64_t i = threadIdx.x; i < e.nb; i += blockDim.x) bit_off[e.bbase + i] = off;
-    if (threadIdx.x == 0) {
-        const uint64_t p = pos[e.bbase + e.nb] - pos[e.bbase] + e.rice_word * 64;
-        atomicOr(&words[p >> 6], 1ull << (p & 63));
-    }
-}
-
 struct EfScalars {
     uint64_t bpk;
     long long min_delta;
     long long min_diff;
     uint64_t total_bits;
 };
+constexpr long long kEfMinStart = 0x3FFFFFFFFFFFFFFFll;
 
-// One workgroup per set: bits_per_key_fixed_point (IEEE double, DoubleEF.hpp:144)
-// and the two minima (DoubleEF.hpp:146-179) over the set's buckets, with key
-// counts and bit positions relative to the set.
+// Workgroups (set, part): bit offset of every bucket of the set inside the global
+// Golomb-Rice buffer, the sentinel bit after the set's last bucket (appendFixed(1, 1),
+// SIMDRecSplit.hpp:810), and the start values of the set's minima.  Like the two
+// Elias-Fano kernels below, gridDim.y workgroups stride over a set's buckets: one
+// workgroup took 217 us for the Elias-Fano arrays of 10,000 buckets.
+__global__ __launch_bounds__(256) void k_set_offsets(const SetEnc *__restrict__ sets, const uint64_t *__restrict__ pos,
+                                                     long long *__restrict__ bit_off,
+                                                     unsigned long long *__restrict__ words, EfScalars *__restrict__ efs,
+                                                     const uint32_t *__restrict__ stop = nullptr) {
+    if (stop && (*stop & kErrStopEncode)) return;
+    const SetEnc e = sets[blockIdx.x];
+    const long long off = (long long)(e.rice_word * 64) - (long long)pos[e.bbase];
+    for (uint64_t i = (uint64_t)blockIdx.y * blockDim.x + threadIdx.x; i < e.nb; i += (uint64_t)gridDim.y * blockDim.x)
+        bit_off[e.bbase + i] = off;
+    if (threadIdx.x == 0 && blockIdx.y == 0) {
+        const uint64_t p = pos[e.bbase + e.nb] - pos[e.bbase] + e.rice_word * 64;
+        atomicOr(&words[p >> 6], 1ull << (p & 63));
+        efs[blockIdx.x].min_delta = kEfMinStart;
+        efs[blockIdx.x].min_diff = kEfMinStart;
+    }
+}
+
+// Workgroups (set, part): bits_per_key_fixed_point (IEEE double, DoubleEF.hpp:144) and
+// the two minima (DoubleEF.hpp:146-179) over the set's buckets, with key counts and bit
+// positions relative to the set.  The minima start at kEfMinStart (k_set_offsets).
 __global__ __launch_bounds__(256) void k_ef_scalars(const SetEnc *__restrict__ sets, const uint64_t *__restrict__ acc,
                                                     const uint64_t *__restrict__ pos, EfScalars *__restrict__ out) {
     __shared__ uint64_t s_bpk;
@@ -2018,8 +2024,8 @@ __global__ __launch_bounds__(256) void k_ef_scalars(const SetEnc *__restrict__ s
     if (threadIdx.x == 0) s_bpk = (uint64_t)((double)(1ull << 20) * ((double)(ps[nb] - p0) / (double)(cum[nb] - c0)));
     __syncthreads();
     const uint64_t bpk = s_bpk;
-    long long md = 0x3FFFFFFFFFFFFFFFll, mf = 0x3FFFFFFFFFFFFFFFll;
-    for (uint64_t i = 1 + threadIdx.x; i <= nb; i += blockDim.x) {
+    long long md = kEfMinStart, mf = kEfMinStart;
+    for (uint64_t i = 1 + (uint64_t)blockIdx.y * blockDim.x + threadIdx.x; i <= nb; i += (uint64_t)gridDim.y * blockDim.x) {
         const uint64_t ci = cum[i] - c0, cp = cum[i - 1] - c0;
         const long long d = (long long)(ci - cp);
         md = d < md ? d : md;
@@ -2038,14 +2044,16 @@ __global__ __launch_bounds__(256) void k_ef_scalars(const SetEnc *__restrict__ s
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        out[blockIdx.x].bpk = bpk;
-        out[blockIdx.x].min_delta = s_a[0];
-        out[blockIdx.x].min_diff = s_b[0];
-        out[blockIdx.x].total_bits = ps[nb] - p0;
+        atomicMin(&out[blockIdx.x].min_delta, s_a[0]);
+        atomicMin(&out[blockIdx.x].min_diff, s_b[0]);
+        if (blockIdx.y == 0) {
+            out[blockIdx.x].bpk = bpk;
+            out[blockIdx.x].total_bits = ps[nb] - p0;
+        }
     }
 }
 
-// One workgroup per set, DoubleEF.hpp:204-349: lower bits of both sequences
+// Workgroups (set, part), DoubleEF.hpp:204-349: lower bits of both sequences
 // interleaved per bucket, one upper bit per bucket in each upper-bits array, and
 // the jump table (every q-th element: 64-bit head per super block, 16-bit
 // offsets), computed directly from each sampled element's upper-bit position.
@@ -2069,7 +2077,7 @@ __global__ __launch_bounds__(256) void k_ef_fill(const SetEnc *__restrict__ sets
         const uint64_t pv = (uint64_t)((long long)(ps[i] - p0) - (long long)(f.bpk * ci >> 20)) - i * (uint64_t)f.min_diff;
         return (pv >> lp) + i;
     };
-    for (uint64_t i = threadIdx.x; i <= e.nb; i += blockDim.x) {
+    for (uint64_t i = (uint64_t)blockIdx.y * blockDim.x + threadIdx.x; i <= e.nb; i += (uint64_t)gridDim.y * blockDim.x) {
         const uint64_t ci = cum[i] - c0;
         const uint64_t cv = ci - i * (uint64_t)f.min_delta;
         const uint64_t pval = (uint64_t)((long long)(ps[i] - p0) - (long long)(f.bpk * ci >> 20)) - i * (uint64_t)f.min_diff;

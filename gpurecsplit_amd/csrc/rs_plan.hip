@@ -27,11 +27,11 @@ struct PlanMeta {
 };
 
 __global__ __launch_bounds__(256) void k_plan_tiles(KeyTile *__restrict__ tiles, const uint64_t *keys, uint64_t n,
-                                                    uint64_t nb, uint32_t n_tiles) {
+                                                    uint64_t nb, uint32_t n_tiles, uint64_t tile_keys) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_tiles) return;
-    const uint64_t k0 = (uint64_t)t * kTileKeys;
-    tiles[t] = KeyTile{keys, k0, k0 + kTileKeys < n ? k0 + kTileKeys : n, nb, 0};
+    const uint64_t k0 = (uint64_t)t * tile_keys;
+    tiles[t] = KeyTile{keys, k0, k0 + tile_keys < n ? k0 + tile_keys : n, nb, 0};
 }
 
 // Fills p[0, n) with v, n = count ? min(*count + extra, cap) : cap (grid-stride).
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void k_plan_serialize(const PlanMeta *__restri
 
 struct rs_plan {
     int device = 0, num_cus = 0;
-    uint64_t n = 0, nb = 0, bucket = 0;
+    uint64_t n = 0, nb = 0, bucket = 0, tile_keys = 0;
     uint32_t leaf = 0;
     int flags = 0;
     uint8_t *mem = nullptr;  // one device allocation holding every buffer below
@@ -276,7 +276,7 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
     const uint64_t NB = p->nb;
     const uint32_t fill_grid = (uint32_t)p->num_cus * 4;
     // ---- partition (the ordinary build's steps 1-3)
-    k_plan_tiles<<<(p->n_tiles + 255) / 256, 256, 0, s>>>(p->tiles, keys, p->n, NB, p->n_tiles);
+    k_plan_tiles<<<(p->n_tiles + 255) / 256, 256, 0, s>>>(p->tiles, keys, p->n, NB, p->n_tiles, p->tile_keys);
     k_fill<uint32_t><<<fill_grid, 256, 0, s>>>(p->counts, NB, 0u);
     k_fill<uint32_t><<<1, 256, 0, s>>>(p->size_hist, kMaxBucket + 1, 0u);
     k_fill<uint32_t><<<1, 64, 0, s>>>(p->err, 16, 0u);
@@ -417,15 +417,16 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
     scan_level(s, p->bits, false, NB, p->pos, p->scan_tmp);
     k_plan_rice<<<1, 64, 0, s>>>(p->pos, NB, p->cap_rice, p->enc, p->meta, p->err);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->rice, p->cap_rice, 0ull, &p->meta->rice_words, 2);
-    k_set_offsets<<<1, 256, 0, s>>>(p->enc, p->pos, p->bit_off, p->rice, p->err);
+    const dim3 parts(1, ef_parts(NB, 1));
+    k_set_offsets<<<parts, 256, 0, s>>>(p->enc, p->pos, p->bit_off, p->rice, p->efs, p->err);
     k_rice_write<<<(uint32_t)((NB + 3) / 4), 256, 0, s>>>(ca, p->pos, p->bit_off, p->rice);
-    k_ef_scalars<<<1, 256, 0, s>>>(p->enc, p->acc, p->pos, p->efs);
+    k_ef_scalars<<<parts, 256, 0, s>>>(p->enc, p->acc, p->pos, p->efs);
     k_plan_ef<<<1, 64, 0, s>>>(p->efs, p->n, NB, p->cap_lower, p->cap_upper, p->enc, p->meta, p->err);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->lower, p->cap_lower, 0ull, &p->meta->lower_words, 1);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->uc, p->cap_upper, 0ull, &p->meta->uc_words, 1);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->up, p->cap_upper, 0ull, &p->meta->up_words, 1);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->jump, p->cap_jump, 0ull, &p->meta->jump_words, 1);
-    k_ef_fill<<<1, 256, 0, s>>>(p->enc, p->efs, p->acc, p->pos, p->lower, p->uc, p->up, (uint8_t *)p->jump, p->err,
+    k_ef_fill<<<parts, 256, 0, s>>>(p->enc, p->efs, p->acc, p->pos, p->lower, p->uc, p->up, (uint8_t *)p->jump, p->err,
                                 p->err);
     k_plan_serialize<<<1, 256, 0, s>>>(p->meta, p->leaf, p->bucket, p->n, p->rice, p->lower, p->uc, p->up,
                                        (const uint64_t *)p->jump, p->cap_out, p->out, p->out_words, p->err);
@@ -450,7 +451,8 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
         p->tune = tune_for(c, leaf);
         p->blocks = (uint32_t)c->num_cus * (uint32_t)p->tune.blocks_per_cu;
         p->n_waves = p->blocks * 4;
-        p->n_tiles = (uint32_t)((n + kTileKeys - 1) / kTileKeys);
+        p->tile_keys = tile_size(n, p->nb, (uint32_t)p->num_cus);
+        p->n_tiles = (uint32_t)((n + p->tile_keys - 1) / p->tile_keys);
         const uint64_t NB = p->nb;
         const SplitParams P = split_params(leaf);
         // bounds: nodes < n (a tree over m keys has at most m - 1 nodes); descriptors

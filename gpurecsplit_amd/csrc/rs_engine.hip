@@ -127,10 +127,11 @@ struct DeviceCopy {
     int device = 0;
     uint64_t *mem = nullptr;
     uint64_t *rice = nullptr, *lower = nullptr, *upper_c = nullptr, *upper_p = nullptr, *jump = nullptr;
+    ulonglong2 *table = nullptr;  // first key and first descriptor bit of every bucket (nbuckets + 1)
     uint32_t *memo = nullptr;
     uint64_t n_rice = 0, n_lower = 0, n_uc = 0, n_up = 0, n_jump = 0;
-    // The arrays one after another from p on; the memo table at m.
-    void place(uint64_t *p, uint64_t rice_words, const std::array<uint64_t, 4> &ef_words, uint32_t *m) {
+    // The arrays one after another from p on, then the bucket table and the memo.
+    void place(uint64_t *p, uint64_t rice_words, const std::array<uint64_t, 4> &ef_words, uint64_t nb) {
         n_rice = rice_words;
         n_lower = ef_words[0];
         n_uc = ef_words[1];
@@ -141,8 +142,12 @@ struct DeviceCopy {
         upper_c = lower + n_lower;
         upper_p = upper_c + n_uc;
         jump = upper_p + n_up;
-        memo = m;
+        const uint64_t at = (uint64_t)(jump + n_jump - mem);
+        table = (ulonglong2 *)(mem + ((at + 1) & ~uint64_t(1)));  // 16-byte aligned
+        memo = (uint32_t *)(table + nb + 1);
     }
+    // Words of an allocation whose arrays end at word `at`.
+    static uint64_t words(uint64_t at, uint64_t nb) { return ((at + 1) & ~uint64_t(1)) + 2 * (nb + 1) + kMaxBucket / 2; }
 };
 
 void device_copy_free(DeviceCopy *d) {
@@ -1111,8 +1116,10 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     // follow from the scalars: at most 2 lower words per bucket (two widths below 64)
     // and 3 bits per bucket in either upper array (u >> l < 2 (nb + 1)).
     uint64_t ef_cap = 0;
+    // A single set's device copy also takes the bucket table behind them.
+    const uint64_t table_words = device_copy && S == 1 ? 2 * (nbs[0] + 1) + 1 : 0;
     for (size_t i = 0; i < S; i++) ef_cap += 2 * (nbs[i] + 2) + 2 * (3 * (nbs[i] + 1) / 64 + 2) + ef_jump_words(nbs[i]);
-    unsigned long long *result = c->rice.get<unsigned long long>(1 + rice_total + ef_cap);
+    unsigned long long *result = c->rice.get<unsigned long long>(1 + rice_total + ef_cap + table_words);
     HIP_CHECK(hipMemsetAsync(result, 0, (1 + rice_total + ef_cap) * 8, s));
     unsigned long long *rice = result + 1;
     SetEnc *d_enc = c->set_enc.get<SetEnc>(S);
@@ -1178,7 +1185,9 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         throw BuildError(RS_ERR_INTERNAL, "Elias-Fano arrays beyond their bound");
     unsigned long long *d_lower = rice + rice_total, *d_uc = d_lower + tot_lower, *d_up = d_uc + tot_uc;
     uint8_t *d_jump = (uint8_t *)(d_up + tot_up);
-    k_ef_fill<<<parts, 256, 0, s>>>(d_enc, d_efs, acc, pos, d_lower, d_uc, d_up, d_jump, (uint32_t *)result);
+    const uint64_t total_words = 1 + rice_total + tot_lower + tot_uc + tot_up + tot_jump;
+    ulonglong2 *d_table = table_words ? (ulonglong2 *)(result + ((total_words + 1) & ~uint64_t(1))) : nullptr;
+    k_ef_fill<<<parts, 256, 0, s>>>(d_enc, d_efs, acc, pos, d_lower, d_uc, d_up, d_jump, (uint32_t *)result, d_table);
     HIP_CHECK(hipGetLastError());
     const int e_enc_end = ev_record(c);
 
@@ -1225,7 +1234,6 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     // One copy of all arrays of all sets into the context's pinned staging (a copy into
     // fresh pageable memory took 27 ms longer for the 126 MB of 4096 sets of 590M
     // keys); the handles take their words from there.
-    const uint64_t total_words = 1 + rice_total + tot_lower + tot_uc + tot_up + tot_jump;
     const uint64_t *h_result = c->h_result.get(8 * total_words);
     const uint64_t *h_rice = h_result + 1, *h_lower = h_rice + rice_total, *h_uc = h_lower + tot_lower,
                    *h_up = h_uc + tot_uc, *h_jump = h_up + tot_up;
@@ -1234,9 +1242,9 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
     if (device_copy && S == 1) {
         dc = new DeviceCopy();
         dc->device = c->device;
-        HIP_CHECK(hipMalloc(&dc->mem, total_words * 8 + kMaxBucket * 4));
-        dc->place(dc->mem + 1, rice_total, ef_words[0], (uint32_t *)(dc->mem + total_words));
-        HIP_CHECK(hipMemcpyAsync(dc->mem, result, total_words * 8, hipMemcpyDeviceToDevice, s));
+        HIP_CHECK(hipMalloc(&dc->mem, DeviceCopy::words(total_words, NB) * 8));
+        dc->place(dc->mem + 1, rice_total, ef_words[0], NB);
+        HIP_CHECK(hipMemcpyAsync(dc->mem, result, ((uint64_t *)dc->memo - dc->mem) * 8, hipMemcpyDeviceToDevice, s));
         HIP_CHECK(hipMemcpyAsync(dc->memo, memo, kMaxBucket * 4, hipMemcpyDeviceToDevice, s));
     }
     HIP_CHECK(hipStreamSynchronize(s));
@@ -1482,15 +1490,19 @@ static const DeviceCopy *device_copy_of(rs_ctx *c, rs_mphf *h) {
     };
     try {
         const uint64_t words = h->rice_words + ef.lower_bits.size() + ef.upper_cum.size() + ef.upper_pos.size() + ef.jump.size();
-        HIP_CHECK(hipMalloc(&dc->mem, words * 8 + kMaxBucket * 4));
+        HIP_CHECK(hipMalloc(&dc->mem, DeviceCopy::words(words, h->nbuckets) * 8));
         dc->place(dc->mem, h->rice_words, {ef.lower_bits.size(), ef.upper_cum.size(), ef.upper_pos.size(), ef.jump.size()},
-                  (uint32_t *)(dc->mem + words));
+                  h->nbuckets);
         up(dc->rice, h->rice.data(), dc->n_rice);
         up(dc->lower, ef.lower_bits.data(), dc->n_lower);
         up(dc->upper_c, ef.upper_cum.data(), dc->n_uc);
         up(dc->upper_p, ef.upper_pos.data(), dc->n_up);
         up(dc->jump, ef.jump.data(), dc->n_jump);
         HIP_CHECK(hipMemcpyAsync(dc->memo, h->memo->data(), kMaxBucket * 4, hipMemcpyHostToDevice, c->stream));
+        EfArgs e{dc->lower, dc->upper_c, dc->upper_p, dc->jump, dc->n_lower, dc->n_uc, dc->n_up, dc->n_jump,
+                 h->nbuckets, ef.bits_per_key_fixed_point, ef.l_cum_keys, ef.l_position, ef.cum_keys_min_delta, ef.min_diff};
+        k_bucket_table<<<(uint32_t)((h->nbuckets + 256) / 256), 256, 0, c->stream>>>(e, dc->table);
+        HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipStreamSynchronize(c->stream));
     } catch (...) {
         device_copy_free(dc);
@@ -1752,26 +1764,18 @@ int rs_query_device(rs_ctx *c, const rs_mphf *h, const uint64_t *d_keys, size_t 
         const DeviceCopy *dc = device_copy_of(c, const_cast<rs_mphf *>(h));
         QueryArgs q{};
         q.rice = dc->rice;
-        q.lower = dc->lower;
-        q.upper_c = dc->upper_c;
-        q.upper_p = dc->upper_p;
-        q.jump = dc->jump;
-        q.memo = dc->memo;
         q.n_rice = dc->n_rice;
-        q.n_lower = dc->n_lower;
-        q.n_uc = dc->n_uc;
-        q.n_up = dc->n_up;
-        q.n_jump = dc->n_jump;
+        q.table = dc->table;
+        q.memo = dc->memo;
         q.keys_count = h->keys_count;
         q.nbuckets = h->nbuckets;
-        q.bpk = h->ef.bits_per_key_fixed_point;
-        q.lc = h->ef.l_cum_keys;
-        q.lp = h->ef.l_position;
-        q.min_delta = h->ef.cum_keys_min_delta;
-        q.min_diff = h->ef.min_diff;
         q.P = h->P;
         q.rotate = h->rotate;
-        k_query<<<(n + 255) / 256, 256, 0, c->stream>>>(q, d_keys, n, d_out);
+        auto magic = [](uint32_t d) { return (uint32_t)(((uint64_t(1) << 32) + d - 1) / d); };
+        q.upper_magic = magic(h->P.upper);
+        q.lower_magic = magic(h->P.lower);
+        q.leaf_magic = magic(h->P.leaf);
+        k_query<<<(n + 255) / 256, 256, 0, c->stream>>>(q, (const Two64 *)d_keys, n, d_out);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipStreamSynchronize(c->stream));
     });

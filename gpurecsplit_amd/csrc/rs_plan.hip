@@ -426,8 +426,8 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->uc, p->cap_upper, 0ull, &p->meta->uc_words, 1);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->up, p->cap_upper, 0ull, &p->meta->up_words, 1);
     k_fill<unsigned long long><<<fill_grid, 256, 0, s>>>(p->jump, p->cap_jump, 0ull, &p->meta->jump_words, 1);
-    k_ef_fill<<<parts, 256, 0, s>>>(p->enc, p->efs, p->acc, p->pos, p->lower, p->uc, p->up, (uint8_t *)p->jump, p->err,
-                                p->err);
+    k_ef_fill<<<parts, 256, 0, s>>>(p->enc, p->efs, p->acc, p->pos, p->lower, p->uc, p->up, (uint8_t *)p->jump,
+                                    p->err, nullptr, p->err);
     k_plan_serialize<<<1, 256, 0, s>>>(p->meta, p->leaf, p->bucket, p->n, p->rice, p->lower, p->uc, p->up,
                                        (const uint64_t *)p->jump, p->cap_out, p->out, p->out_words, p->err);
     HIP_CHECK(hipGetLastError());

@@ -312,7 +312,8 @@ using namespace rsa;
 // gK: 64*u-candidate groups per claimed chunk of kind K, hK: helper cap of kind K
 // (0: none), bpc: workgroups of 4 waves per CU, bt: byte table for aggregation
 // levels of mostly full-size nodes, ubt: candidates per lane there, btw / ubtw: the
-// same for 64-bit counters, btl: byte table of positions for rotation leaves).
+// same for 64-bit counters, btl: byte table of positions for rotation leaves, pk:
+// packed parts for aggregation levels, tree: whole trees of small buckets).
 // Fanout-2 nodes need ~40 candidates, so they run one per lane.
 struct Tune {
     // upper aggregation one per lane: its increment-table launches are the levels
@@ -333,7 +334,7 @@ struct Tune {
     int help_cap[kNumKinds] = {2, 0, 0, 0, 0};
     int blocks_per_cu = 8;
     int tree = 1;    // whole trees of small buckets in one kernel
-    int pk = 1;      // packed parts for the full-size nodes of heavy aggregation levels
+    int pk = 1;      // packed parts for the full-size nodes of heavy aggregation levels (2: of levels of any work)
     int bt = 1;      // byte table for the full-size nodes of aggregation levels
     int u_bt = 4;    // candidates in flight per lane in those launches
     int bt_leaf = 1; // byte table of positions for rotation leaves
@@ -360,7 +361,7 @@ static Tune parse_tune(const char *env, Tune t = Tune()) {
                 t.u[k[1] - '0'] = v;
             else if (k == "lut") t.lut = v != 0;
             else if (k == "tree") t.tree = v != 0;
-            else if (k == "pk") t.pk = v != 0;
+            else if (k == "pk" && v >= 0 && v <= 2) t.pk = v;
             else if (k == "bt") t.bt = v != 0;
             else if (k == "ubt" && uv) t.u_bt = v;
             else if (k == "btl") t.bt_leaf = v != 0;
@@ -581,6 +582,11 @@ static void launch_sk(hipStream_t s, int u, uint32_t kind, const uint64_t *keys,
 // Packed parts (full-size aggregation nodes) from this Golomb-Rice parameter of the
 // level's full size on: 2.08 * 2^12 = 8,500 expected candidates, sixteen groups of 512.
 constexpr uint32_t kPkMinGolomb = 12;
+// ... and from this many expected evaluations of the level on: a shorter level ends
+// with waves sharing its nodes, in chunks twice the byte table's.  Byte table / packed
+// in ms: 50K keys at l = 15, b = 500 upper (5.7e9) 2.10 / 2.38, lower (1.5e9) 1.01 /
+// 1.12; 200K at l = 14 lower (6e9) 2.08 / 2.26; 500K at l = 13 lower (1.2e10) 5.2 / 4.6.
+constexpr double kPkMinEvals = 1e10;
 
 // Grid of one search level from its size in 4-wave workgroups: the byte-table
 // instance (aggregation levels with 32-bit counters whose nodes are mostly of the
@@ -593,14 +599,22 @@ struct SearchShape {
 };
 static SearchShape search_shape(const Tune &tn, uint32_t kind, bool wide, bool lut, bool r64, bool mostly_full,
                                 uint32_t blocks4, uint32_t full_blocks4, uint32_t num_cus, uint32_t leaf_size,
-                                uint32_t golomb, double nodes) {
-    if (tn.pk && (kind == kUpper || kind == kLower) && lut && !r64 && mostly_full && golomb >= kPkMinGolomb) {
-        // eight independent candidates per lane keep a SIMD busy with few waves, and
-        // waves that only help on other waves' nodes cost more than they give: levels
-        // of fewer nodes than the grid has waves run four waves per SIMD (100K keys at
-        // l = 16: lower 10.3 -> 9.2 ms, upper 5.7 -> 5.2; 1M keys: upper 33.7 -> 32.9;
-        // its lower level of 9,100 nodes keeps the grid, 66.4 ms against 71.0)
-        const uint32_t b = nodes < 4.0 * full_blocks4 ? std::min(blocks4, 4 * num_cus) : blocks4;
+                                uint32_t golomb, double nodes, double evals) {
+    if ((tn.pk > 1 || (tn.pk && evals >= kPkMinEvals)) && (kind == kUpper || kind == kLower) && lut && !r64 &&
+        mostly_full && golomb >= kPkMinGolomb) {
+        // Eight independent candidates per lane keep a SIMD busy with few waves, and more
+        // waves make each node's search longer and its helpers' work past the hit more.
+        // Levels of small nodes therefore run four waves per SIMD.  Lower levels in ms at
+        // eight / four waves and by the byte table: 3M keys at l = 14, b = 100 (2.9e6
+        // evaluations per node) 31.7 / 16.8 / 20.1; 1M at l = 15, b = 500 21.5 / 8.3 /
+        // 11.0; 2M at l = 13, b = 2000 26.7 / 12.2 / 14.5.  At 4.3e7 per node (1M keys
+        // at l = 16) the full grid is the faster, 65.8 / 70.9 / 76.8, unless the level
+        // has fewer nodes than the grid has waves (its upper level, 2,000 nodes, 33.7 /
+        // 32.9); below an eighth of them three are best (100K keys: 950 lower nodes
+        // 10.3, 9.25 and 8.9 on the grid, four and three, 200 upper nodes 5.7, 5.2, 4.9).
+        const double grid_waves = 4.0 * full_blocks4;
+        const uint32_t per_simd = 8 * nodes < grid_waves ? 3 : nodes < grid_waves || evals < 1.5e7 * nodes ? 4 : 8;
+        const uint32_t b = per_simd == 8 ? blocks4 : std::min(blocks4, per_simd * num_cus);
         return {b, b * 4, false, true};
     }
     const bool aggr = tn.bt && (kind == kUpper || kind == kLower) && lut && (!wide || tn.bt_wide) && mostly_full;
@@ -1026,7 +1040,7 @@ static std::vector<rs_mphf *> build_sets(rs_ctx *c, const std::vector<const uint
         }
         const SearchShape sh =
             search_shape(tn, kind, wide, lut, r64, 2 * cen.full[l] >= cnt, lblocks, blocks, (uint32_t)c->num_cus, leaf,
-                         lds ? golomb_param(hmemo, a.lut_entries) : 0, (double)cnt);
+                         lds ? golomb_param(hmemo, a.lut_entries) : 0, (double)cnt, cen.evals[l]);
         a.bt_m = sh.bt || sh.pk ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
         a.n_waves = sh.waves;
         if (sh.pk) {

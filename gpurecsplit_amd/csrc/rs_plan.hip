@@ -219,6 +219,7 @@ struct rs_plan {
     std::vector<char> likely;   // ... and whether a bucket of the likely sizes has it
     std::vector<uint32_t> level_blocks;  // ... and its search grid (expected work)
     std::vector<double> level_nodes;     // ... and its expected nodes
+    std::vector<double> level_evals;     // ... and their evaluations
     std::vector<char> mostly_full;       // ... and whether most of its nodes are of full size
     uint32_t likely_max_bucket = 0;  // bucket sizes above this are vanishingly rare
     bool tree = false;               // buckets run as whole trees (k_tree)
@@ -384,7 +385,8 @@ static void plan_enqueue(rs_plan *p, const uint64_t *keys, hipStream_t s) {
         }
         const SearchShape sh =
             search_shape(tn, kind, wide, lut, r64, p->mostly_full[li] != 0, blocks, p->blocks, (uint32_t)p->num_cus, P.leaf,
-                         lds ? golomb_param(golomb_memo(P.leaf), a.lut_entries) : 0, p->level_nodes[li]);
+                         lds ? golomb_param(golomb_memo(P.leaf), a.lut_entries) : 0, p->level_nodes[li],
+                         p->level_evals[li]);
         a.bt_m = sh.bt || sh.pk ? (kind == kLeafRot ? P.leaf : a.lut_entries) : 0;
         a.n_waves = sh.waves;
         k_level_init<<<likely ? fill_grid : 4, 256, 0, s>>>(p->state, p->running, p->ctl, sh.waves, p->list_count,
@@ -548,6 +550,7 @@ int rs_plan_create(rs_ctx *c, size_t n, uint32_t leaf, size_t bucket, int flags,
                 p->likely.push_back(lik ? 1 : 0);
                 p->level_blocks.push_back(rsa::level_blocks(e * (double)NB, cnt * (double)NB, p->blocks));
                 p->level_nodes.push_back(cnt * (double)NB);
+                p->level_evals.push_back(e * (double)NB);
                 p->mostly_full.push_back(2 * nfull >= cnt ? 1 : 0);
             }
         }

@@ -666,9 +666,11 @@ struct TreeWork {
 // of `tail` (a wave hashes 64 keys in about 50 cycles), nor before a bucket's own
 // evaluations (shared by four waves where buckets are few).  The level kernels'
 // launches, syncs and per-node atomics cost about 0.6 ms and 18 ns per node beside the
-// evaluations that both do.  Both sides measured at 1K to 3M keys, l = 4..16: 1M keys
-// at l = 8, b = 100 4.4 ms by levels, 1.1 as trees; l = 12, b = 100 4.4 and 2.4;
-// 1M keys at l = 14, b = 20 8.6 and 5.9, but 100K of them 2.0 and 2.4.
+// evaluations that both do.  Both sides measured, levels / trees in ms, at 100K to 10M
+// keys and l = 4..16: 1M keys at l = 8, b = 100 3.9 / 0.8; 10M at l = 12, b = 100
+// 20.5 / 11.9; 1.8M at l = 12, b = 200 8.2 / 6.1; 1M at l = 14, b = 20 8.5 / 4.7.  The
+// other way: 100K at l = 14, b = 20 1.8 / 2.1, 1M at l = 13, b = 50 4.3 / 5.8, 300K at
+// l = 14, b = 100 4.7 / 12.1, 1M at l = 16, b = 20 19 / 28.
 constexpr uint32_t kTreeMaxBucket = 512;
 static bool tree_fits(const Tune &tn, const AggrLayout &up, const AggrLayout &lo, uint32_t max_bucket,
                       const TreeWork &w, double buckets, uint32_t num_cus) {

@@ -200,7 +200,7 @@ struct TreeItem {
     uint32_t slot;
 };
 
-// UL: candidates per lane of the lower aggregation level and the leaves.  TEAM: a
+// UL: candidates per lane of the leaves and of heavy aggregation nodes.  TEAM: a
 // workgroup per bucket whose waves take the nodes of one tree depth after another
 // (few buckets: more waves than one per bucket); otherwise a wave per bucket, node
 // by node in preorder.
@@ -283,13 +283,17 @@ __global__ __launch_bounds__(TEAM ? 512 : 256, TEAM ? 2 : 4) void k_tree(TreeArg
             uint32_t T = 0;
             for (uint32_t p = 0; p + 1 < fan; p++) T |= unit << (p * fb);
             const uint32_t cmask = (1u << ((fan - 1) * fb)) - 1;  // at most 31 bits
-            if (up)
-                x = tree_groups<1>(1, m, sh, work, [&](uint64_t u0) {
-                    return group_aggr<1, false, true, kKeysLds, R64>(kp, m, seed0, fb, magic, T, cmask, up_hi, 2, u0);
+            const uint32_t hi = up ? up_hi : lo_hi;
+            // UL candidates per lane from about 500 expected candidates on, on both levels
+            // (1.8M keys at l = 12, b = 200, upper level one per lane 10.0 ms, this 6.1),
+            // one below (a pass of UL tests 64 UL at once)
+            if (UL > 1 && gol[m] >= 8)
+                x = tree_groups<UL>(1, m, sh, work, [&](uint64_t u0) {
+                    return group_aggr<UL, false, true, kKeysLds, R64>(kp, m, seed0, fb, magic, T, cmask, hi, 2, u0);
                 });
             else
-                x = tree_groups<UL>(1, m, sh, work, [&](uint64_t u0) {
-                    return group_aggr<UL, false, true, kKeysLds, R64>(kp, m, seed0, fb, magic, T, cmask, lo_hi, 2, u0);
+                x = tree_groups<1>(1, m, sh, work, [&](uint64_t u0) {
+                    return group_aggr<1, false, true, kKeysLds, R64>(kp, m, seed0, fb, magic, T, cmask, hi, 2, u0);
                 });
         } else {
             const bool odd_key = lane < m && (kp[lane < m ? lane : 0] & 1) != 0;

@@ -671,12 +671,26 @@ struct TreeWork {
 // 20.5 / 11.9; 1.8M at l = 12, b = 200 8.2 / 6.1; 1M at l = 14, b = 20 8.5 / 4.7.  The
 // other way: 100K at l = 14, b = 20 1.8 / 2.1, 1M at l = 13, b = 50 4.3 / 5.8, 300K at
 // l = 14, b = 100 4.7 / 12.1, 1M at l = 16, b = 20 19 / 28.
+// Larger buckets (up to kMaxBucket, 132 KB of LDS at most) take a workgroup each.  Its
+// eight waves share the few nodes near the root, but a node's keys are ordered by one
+// wave and few workgroups share a CU, so they pay only where no search is long: the
+// bound is under 0.32 ms on every shape that gained and over 0.81 ms on every one that
+// lost.  Levels / trees in ms at 3K, 200K and 2M keys: l = 4, b = 1000 1.66 / 0.63,
+// 3.95 / 0.78, 16.0 / 2.8; l = 8, b = 2000 1.36 / 0.87, 3.36 / 1.27, 8.8 / 4.3; l = 10,
+// b = 500 0.87 / 0.43, 2.06 / 0.82, 6.0 / 4.7; but l = 11, b = 500 0.93 / 1.25, 2.7 /
+// 2.8, 8.5 / 15.6 and l = 12, b = 1000 1.35 / 2.08, 3.3 / 4.5, 9.9 / 18.8.  Two waves
+// per SIMD also hash slower, so the evaluations must stay below what the levels'
+// launches and nodes cost, at 1.3 ps each: 1M keys at l = 10, b = 500 without rotations
+// (3.8e9) 4.1 / 4.8, 2M with (2.0e9) 6.0 / 4.7 (the line lies between 0.9 and 2.6 ps).
 constexpr uint32_t kTreeMaxBucket = 512;
 static bool tree_fits(const Tune &tn, const AggrLayout &up, const AggrLayout &lo, uint32_t max_bucket,
                       const TreeWork &w, double buckets, uint32_t num_cus) {
-    if (!tn.tree || up.wide || lo.wide || max_bucket > kTreeMaxBucket) return false;
-    const double chain = w.evals / buckets / (buckets <= 8.0 * num_cus ? 4 : 1);
-    return 0.32e-9 * std::max(w.tail, chain) <= 0.6e-3 + 18e-9 * w.nodes;
+    if (!tn.tree || up.wide || lo.wide) return false;
+    const bool large = max_bucket > kTreeMaxBucket;
+    const double chain = w.evals / buckets / (large || buckets <= 8.0 * num_cus ? 4 : 1);
+    const double bound = 0.32e-9 * std::max(w.tail, chain);
+    const double saved = 0.6e-3 + 18e-9 * w.nodes;
+    return large ? bound <= 0.5e-3 && 1.3e-12 * w.evals <= saved : bound <= saved;
 }
 
 // Candidates per lane of the lower level and the leaves: one where a node's expected
@@ -693,10 +707,10 @@ static void launch_tree_u(hipStream_t s, const TreeArgs &a, uint32_t blocks, uin
     }
 }
 static uint32_t launch_tree(hipStream_t s, TreeArgs a, bool r64, uint32_t num_cus) {
-    // a workgroup per bucket while one wave per bucket would not fill the SIMDs
-    // a launch for oversized buckets only (cap above kTreeMaxBucket) always does
+    // a workgroup per bucket while one wave per bucket would not fill the SIMDs, and
+    // for buckets above kTreeMaxBucket, whose LDS leaves room for few workgroups
     const bool team = a.nb <= 8 * num_cus || a.cap > kTreeMaxBucket;
-    const uint32_t wpg = team && a.nb <= 2 * num_cus ? 8 : 4;
+    const uint32_t wpg = team && (a.nb <= 2 * num_cus || a.cap > kTreeMaxBucket) ? 8 : 4;
     const TreeLds l = tree_lds(a.P, a.rotate != 0, a.cap, wpg, team);
     a.scratch = l.scratch;
     a.queue = l.queue;

@@ -4,15 +4,16 @@
 // Pipeline of one build (all on one HIP stream; three small device->host reads):
 //   1. bucket histogram, per-bucket node counts, size histogram, scans
 //      -> read the size histogram: reject buckets >= 3000 keys, size the node lists
-//   2. scatter `second` by bucket, sort each bucket in LDS (detects equal keys)
-//      -> read the error flag
-//   3. expand every bucket's split tree into per-phase node lists
-//   4. per phase (fanout-2 depth 0, 1, ..., upper aggregation, lower aggregation,
-//      rotation leaves, brute-force leaves): persistent seed-search kernel, then
-//      partition of the keys between the children
-//   5. per-bucket descriptor lengths, scan -> read the total bit count
-//   6. Golomb-Rice write; Elias-Fano scalars -> read them; Elias-Fano fill
-//   7. copy the structure to the host (and keep a device copy for queries)
+//   2. scatter `second` by bucket
+//   3. buckets whose searches are short (tree_fits): k_tree searches and splits a
+//      bucket's whole tree with its keys in LDS and finds equal keys.  Otherwise:
+//      sort each bucket in LDS (detects equal keys), expand the split trees into
+//      per-phase node lists, and per phase (fanout-2 depth 0, 1, ..., upper
+//      aggregation, lower aggregation, rotation leaves, brute-force leaves) run the
+//      persistent seed-search kernel, then partition the keys between the children
+//   4. per-bucket descriptor lengths, scan -> read the total bit count
+//   5. Golomb-Rice write; Elias-Fano scalars -> read them; Elias-Fano fill
+//   6. copy the structure to the host (and keep a device copy for queries)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -622,11 +623,12 @@ static SearchShape search_shape(const Tune &tn, uint32_t kind, bool wide, bool l
     const uint32_t wpg = bt_threads((int)kind) / 64;  // waves per workgroup
     // A leaf level of fewer waves than half a byte-table workgroup per CU would
     // put its waves on a few CUs (sharing their SIMDs) while others idle; it runs
-    // the 4-wave workgroups instead.  Measured rotation levels: 828 waves (10K keys,
-    // l = 16) 0.84 -> 0.67 ms, 984 waves (100K keys, l = 12) 0.41 -> 0.29 ms; at
-    // 2612 waves (100K keys, l = 16) the byte table is faster (2.32 against 2.53 ms).
-    // Small aggregation levels keep the byte table, whose instruction savings
-    // outweigh that (10K keys at l = 16: upper 1.68 ms with it, 2.54 ms without).
+    // the 4-wave workgroups instead.  Measured on rotation levels while those of 12 and
+    // 16 keys ran the table (they are searched in stages by now): 828 waves 0.84 ->
+    // 0.67 ms, 984 waves 0.41 -> 0.29 ms; at 2612 waves the table was the faster (2.32
+    // against 2.53 ms).  Small aggregation levels keep the byte table, whose
+    // instruction savings outweigh that (10K keys at l = 16: upper 1.68 ms with it,
+    // 2.54 ms without).
     const bool fills = (uint64_t)blocks4 * 4 * 2 >= (uint64_t)num_cus * wpg;
     if (!((aggr || (leaf && fills)) && !r64)) return {blocks4, blocks4 * 4, false, false};
     const uint32_t g = std::max<uint32_t>(1, std::min((blocks4 * 4 + wpg - 1) / wpg, full_blocks4 * 4 / wpg));
@@ -671,6 +673,10 @@ struct TreeWork {
 // 20.5 / 11.9; 1.8M at l = 12, b = 200 8.2 / 6.1; 1M at l = 14, b = 20 8.5 / 4.7.  The
 // other way: 100K at l = 14, b = 20 1.8 / 2.1, 1M at l = 13, b = 50 4.3 / 5.8, 300K at
 // l = 14, b = 100 4.7 / 12.1, 1M at l = 16, b = 20 19 / 28.
+// Level kernels batch their tickets on lists of millions of nodes, so what a node costs
+// them stops growing there (15M nodes of a build), while the tree kernel's slower
+// hashing (0.175 ps per expected evaluation) does not: l = 12, b = 100 at 10M, 50M, 100M
+// and 300M keys 20.8 / 12.2, 63 / 57, 118 / 113, 296 / 332; 100M at l = 8 66 / 44.
 // Larger buckets (up to kMaxBucket, 132 KB of LDS at most) take a workgroup each.  Its
 // eight waves share the few nodes near the root, but a node's keys are ordered by one
 // wave and few workgroups share a CU, so they pay only where no search is long: the
@@ -682,6 +688,9 @@ struct TreeWork {
 // per SIMD also hash slower, so the evaluations must stay below what the levels'
 // launches and nodes cost, at 1.3 ps each: 1M keys at l = 10, b = 500 without rotations
 // (3.8e9) 4.1 / 4.8, 2M with (2.0e9) 6.0 / 4.7 (the line lies between 0.9 and 2.6 ps).
+// They are also left to the levels past the sizes at which they gained (5M keys at
+// l = 4, 8 and 10, b = 500: 26.5 / 5.6, 13.4 / 5.6, 11.5 / 11.2): 100M at l = 8, b = 1000
+// 63 / 110.
 constexpr uint32_t kTreeMaxBucket = 512;
 static bool tree_fits(const Tune &tn, const AggrLayout &up, const AggrLayout &lo, uint32_t max_bucket,
                       const TreeWork &w, double buckets, uint32_t num_cus) {
@@ -689,8 +698,9 @@ static bool tree_fits(const Tune &tn, const AggrLayout &up, const AggrLayout &lo
     const bool large = max_bucket > kTreeMaxBucket;
     const double chain = w.evals / buckets / (large || buckets <= 8.0 * num_cus ? 4 : 1);
     const double bound = 0.32e-9 * std::max(w.tail, chain);
-    const double saved = 0.6e-3 + 18e-9 * w.nodes;
-    return large ? bound <= 0.5e-3 && 1.3e-12 * w.evals <= saved : bound <= saved;
+    if (large)
+        return bound <= 0.5e-3 && w.nodes <= 2.6e6 && w.evals <= 7e9 && 1.3e-12 * w.evals <= 0.6e-3 + 18e-9 * w.nodes;
+    return bound <= 0.6e-3 + 18e-9 * w.nodes && 1.75e-13 * w.evals <= 0.6e-3 + 18e-9 * std::min(w.nodes, 15e6);
 }
 
 // Candidates per lane of the lower level and the leaves: one where a node's expected

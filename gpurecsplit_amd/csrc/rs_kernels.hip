@@ -18,6 +18,7 @@
 // node's result is the atomic minimum over all chunks, and a chunk is only
 // skipped once its first seed is not below that minimum, so the result is the
 // lowest valid seed.  Waves with no fresh node help the nodes still running.
+// (Buckets whose searches are short skip the levels: k_tree, rs_tree.hip.)
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -721,8 +722,9 @@ __device__ __forceinline__ uint64_t group_aggr_bt(const uint64_t *__restrict__ k
 // wave-uniform S_j: two adds, xors and multiplies per key serve eight candidates.
 // The parts of four keys share a register (one byte each), and one dot product adds
 // their squares to the candidate's sum.  A candidate whose counts all equal `unit`
-// has the sum unit * (0 + 1 + 4 + ... + (fan - 1)^2); 0.1 to 0.3% of the others
-// have it too, so every candidate with that sum is counted exactly (lane per key).
+// has the sum unit * (0 + 1 + 4 + ... + (fan - 1)^2); 0.12% (l = 24) to
+// 0.65% (l = 13) of the others have it too, so every candidate with that sum is
+// counted exactly (lane per key).
 //
 // About 7 vector instructions per evaluation and no LDS, against 8 instructions and
 // one random byte read of a 64 KiB LDS table (the byte-table instance), whose bank

@@ -75,7 +75,9 @@ typedef struct rs_build_stats {
     double partition_ms;      /* histogram + scans + scatter + per-bucket sort */
     double search_ms[8];      /* search kernels: [0] fanout-2 levels, [1] upper
                                  aggregation, [2] lower aggregation, [3] rotation
-                                 leaves, [4] brute-force leaves */
+                                 leaves, [4] brute-force leaves; a build that runs
+                                 whole trees in one kernel divides that kernel's time
+                                 by the kinds' executed evaluations */
     double split_ms;          /* partition of keys between tree levels */
     double encode_ms;         /* Golomb-Rice + Elias-Fano */
     uint64_t evals[8];        /* algorithmic key-seed evaluations per kind (same index) */
@@ -99,7 +101,8 @@ typedef struct rs_build_stats {
      * leaf (each pass over its L keys tests L rotations, i.e. L seeds) */
     uint64_t seeds[8];
     /* per kind: the most persistent waves a launch of that kind ran with (levels
-     * of little expected work run on fewer than search_waves) */
+     * of little expected work run on fewer than search_waves; a build by whole trees
+     * gives that kernel's waves for every kind with nodes) */
     uint32_t kind_waves[8];
 } rs_build_stats;
 

@@ -52,8 +52,8 @@ KINDS = ["fanout2", "upper_aggr", "lower_aggr", "leaf_rotation", "leaf_bruteforc
 # HBM bytes per launch of the search kernels at the plain l = 16 workload, from
 # two rocprofv3 --pmc runs (FETCH_SIZE scaled x2.0, WRITE_SIZE x1.0: the factors of
 # a 256 MiB copy probe); the profile summaries under profiles/ give the commands.
-# Most of it is register spills written around chunk claims, not key traffic.
-TRAFFIC_BYTES = {"lower_aggr": 15.90e9, "upper_aggr": 10.40e9, "leaf_rotation": 12.20e9}
+# Most of the aggregation levels' is register spills around the packed claims.
+TRAFFIC_BYTES = {"lower_aggr": 226.05e9, "upper_aggr": 34.98e9, "leaf_rotation": 1.71e9}
 
 
 def log(msg: str):
